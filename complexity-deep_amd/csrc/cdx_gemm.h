@@ -174,11 +174,6 @@ __device__ __forceinline__ int xcd_remap(int b, int tiles) {
   return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + k;
 }
 
-// g * sigmoid(g) with the hardware reciprocal (1 ulp) in place of an IEEE division,
-// which costs about ten vector instructions per element; the result is rounded to
-// bf16 afterwards.  exp(-g) overflowing to +inf gives rcp = 0 and silu = -0.
-__device__ __forceinline__ float silu_f32(float g) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)); }
-
 // Four bf16 bias values (8 bytes) as fp32, each clamped to [lo, hi] (the clamp on the
 // mu parameter, core/layer.py:60, applied where the epilogue reads it).
 __device__ __forceinline__ float4 load_bias4(const uint16_t* src, float lo, float hi) {

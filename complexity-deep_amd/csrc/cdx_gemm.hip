@@ -14,9 +14,11 @@
 //                        producer of the next layer's mu operand (the parameter is
 //                        read and clamped in the epilogue)
 //   cdx_linear_fwd       y = x @ W^T (the tied LM head)
+// Products of up to 64 rows (a generation step) run on the skinny kernels (cdx_skinny.h).
 #include <type_traits>
 
 #include "cdx_gemm_persist.h"
+#include "cdx_skinny.h"
 
 namespace cdx {
 namespace {
@@ -102,6 +104,30 @@ int launch(GemmParams p, hipStream_t s, const char* name) {
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// x [M][ldx] times w [N][ldw] over K columns, for the skinny kernels.
+SkinnyParams skinny_params(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, int64_t M, int32_t K,
+                           int32_t N, uint16_t* c, int64_t ldc) {
+  SkinnyParams p{};
+  p.a = p.a2 = x;
+  p.lda = p.lda2 = ldx;
+  p.b = p.b2 = w;
+  p.ldb = ldw;
+  p.M = (int32_t)M;
+  p.N = N;
+  p.K = p.k_split = K;
+  p.c = c;
+  p.ldc = ldc;
+  return p;
+}
+
+// Adds a second source of H columns (mu and its weights).
+void skinny_second(SkinnyParams& p, const uint16_t* mu, int64_t ldmu, const uint16_t* w_mu, int32_t H) {
+  p.a2 = mu;
+  p.lda2 = ldmu;
+  p.b2 = w_mu;
+  p.K += H;
+}
+
 }  // namespace
 }  // namespace cdx
 
@@ -127,6 +153,11 @@ extern "C" int cdx_mu_qkv_fwd(const uint16_t* x, int64_t ldx, const uint16_t* mu
   if (!x || !w || !out || (mu && !w_mu)) return fail(CDX_EINVAL, "%s: null pointer", name);
   if (!aligned16(x) || !aligned16(w) || !aligned16(out) || (mu && (!aligned16(mu) || !aligned16(w_mu))))
     return fail(CDX_EUNSUPPORTED, "%s: pointers must be 16-byte aligned", name);
+  if (skinny_fits(M, N)) {
+    SkinnyParams sp = skinny_params(x, ldx, w, ldw, M, H, N, out, ldo);
+    if (mu) skinny_second(sp, mu, ldmu, w_mu, H);
+    return skinny_gemm(sp, SkinnyEpi::kStore, reinterpret_cast<hipStream_t>(stream), name);
+  }
   GemmParams p{};
   p.a = x;
   p.lda = ldx;
@@ -179,6 +210,9 @@ int moe_swiglu(const uint16_t* x, int64_t T, int32_t H, int32_t Ie, int32_t E, i
   if (blocks * 2 * P * (int64_t)H * 2 > (int64_t)UINT32_MAX)
     return fail(CDX_EUNSUPPORTED, "%s: the gate/up weights must fit 4 GB (E=%d, P=%d, H=%d)", name, E, P, H);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (T <= kSkinnyRows)
+    return skinny_moe(x, (int32_t)T, H, P, E, has_shared != 0, perm, offsets, w_gu, w_down, inter, out, residual, s,
+                      name);
   const int32_t mt = (int32_t)(cdiv(T, kBM) + E);
 
   // Pass 1: gathered rows x[perm] times the gate/up rows of the shared block and the
@@ -495,6 +529,15 @@ extern "C" int cdx_mu_guidance_fwd(const uint16_t* h, int64_t T, int32_t H, cons
   if (!h || !w || !mu || !out) return fail(CDX_EINVAL, "%s: null pointer", name);
   if (!aligned16(h) || !aligned16(w) || !aligned16(mu) || !aligned16(out))
     return fail(CDX_EUNSUPPORTED, "%s: pointers must be 16-byte aligned", name);
+  if (skinny_fits(T, H)) {
+    SkinnyParams sp = skinny_params(h, H, w, H, T, H, H, out, ldo);
+    sp.bias = mu;
+    sp.bias_lo = mu_lo;
+    sp.bias_hi = mu_hi;
+    sp.lo = lo;
+    sp.hi = hi;
+    return skinny_gemm(sp, SkinnyEpi::kBiasClamp, reinterpret_cast<hipStream_t>(stream), name);
+  }
   GemmParams p{};
   p.a = h;
   p.lda = H;
@@ -536,6 +579,9 @@ extern "C" int cdx_linear_fwd(const uint16_t* x, int64_t ldx, const uint16_t* w,
   if (!x || !w || !out) return fail(CDX_EINVAL, "%s: null pointer", name);
   if (!aligned16(x) || !aligned16(w) || !aligned16(out))
     return fail(CDX_EUNSUPPORTED, "%s: pointers must be 16-byte aligned", name);
+  if (skinny_fits(M, N))
+    return skinny_gemm(skinny_params(x, ldx, w, ldw, M, K, N, out, ldo), SkinnyEpi::kStore,
+                       reinterpret_cast<hipStream_t>(stream), name);
   GemmParams p{};
   p.a = x;
   p.lda = ldx;
@@ -570,6 +616,9 @@ extern "C" int cdx_linear_residual_fwd(const uint16_t* x, int64_t ldx, const uin
   if (!x || !w || !residual) return fail(CDX_EINVAL, "%s: null pointer", name);
   if (!aligned16(x) || !aligned16(w) || !aligned16(residual))
     return fail(CDX_EUNSUPPORTED, "%s: pointers must be 16-byte aligned", name);
+  if (skinny_fits(M, N))
+    return skinny_gemm(skinny_params(x, ldx, w, ldw, M, K, N, residual, ldr), SkinnyEpi::kResid,
+                       reinterpret_cast<hipStream_t>(stream), name);
   GemmParams p{};
   p.a = x;
   p.lda = ldx;
