@@ -53,6 +53,14 @@ _SIGNATURES = {
     "cdx_mu_qkv_rope_bcast_fwd": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32,
                                                  _i32, _i32, _vp, _vp, ctypes.c_float, _vp, _i64, _i64, _vp,
                                                  _vp, _vp, _i64, _vp, _vp]),
+    "cdx_few_rows": (_i32, [_i64, _i64]),
+    "cdx_qkv_cache_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i32, _i32, _i32]),
+    "cdx_qkv_cache_fwd": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _i32,
+                                         _vp, _vp, ctypes.c_float, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp,
+                                         ctypes.c_float, _vp, ctypes.c_size_t, _vp]),
+    "cdx_vt_pack": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i32, _vp, _i64, _vp]),
+    "cdx_attention_cache_fwd": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _i64,
+                                               ctypes.c_float, _vp, _vp]),
     "cdx_attention_fwd": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i64, ctypes.c_float,
                                          _vp, _vp]),
     "cdx_mu_guidance_fwd": (ctypes.c_int, [_vp, _i64, _i32, _vp, _vp, ctypes.c_float, ctypes.c_float,
@@ -61,6 +69,7 @@ _SIGNATURES = {
     "cdx_embedding_fwd": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i32, _vp, _vp]),
     "cdx_linear_fwd": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i64, _i32, _i32, _vp, _i64, _vp]),
     "cdx_linear_residual_fwd": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i64, _i32, _i32, _vp, _i64, _vp]),
+    "cdx_linear_accum_fwd": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i64, _i32, _i32, _vp, _i64, _vp]),
     "cdx_hbm_probe": (ctypes.c_int, [_i32, _vp, _vp, _i64, _vp]),
 }
 

@@ -20,8 +20,13 @@ the packed [T, Nq*D + 2*Nkv*D] output.
 ComplexityAttention.forward goes one step further for head dims 32/64/128: the
 per-head QK RMSNorm and RoPE (attention.py:138-155) run in the projection kernel's
 epilogue (cdx_mu_qkv_rope_fwd), which writes q, k, v head-major, in fp32 up to one
-final rounding.  The KV cache, GQA SDPA and o_proj stay PyTorch-ROCm ops in the
-reference's order (attention.py:157-181).
+final rounding.  The few rows of a generation step, and heads of other dims (multiples of
+8 up to 128), go through cdx_qkv_cache_fwd: the product, then one pass that normalises,
+rotates and extends the KV cache.  Without a mask the attention is the causal kernel's,
+with or without a cache: its mask is aligned at the top left, as is_causal=True aligns it
+for more keys than queries (attention.py:168-175), so query i sees keys 0 .. i of the
+cache.  Attention with a mask stays PyTorch-ROCm's SDPA (attention.py:157-181), and o_proj
+of more than a few rows a library GEMM.
 """
 
 from __future__ import annotations
@@ -34,6 +39,7 @@ import torch.nn.functional as F
 
 from . import _native as nat
 from ._grad import forward_only
+from .linear import few_rows, linear, linear_accumulate_
 from .rotary import RotaryEmbedding, apply_rotary_pos_emb
 
 
@@ -233,6 +239,73 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, scale: 
     return out
 
 
+# Queries up to which cdx_qkv_cache_fwd can run the attention itself (keys all cached).
+_ATTEND_ROWS = 16
+
+
+def qkv_cache(x: torch.Tensor, mu: Optional[torch.Tensor], w_x: torch.Tensor, w_mu: torch.Tensor, H: int, nq: int,
+              nkv: int, hd: int, q_norm_w: Optional[torch.Tensor], k_norm_w: Optional[torch.Tensor], eps: float,
+              cos_sin: torch.Tensor, past: Optional[Tuple[torch.Tensor, torch.Tensor]] = None
+              ) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor], torch.Tensor, torch.Tensor]:
+    """(q, attention, k, v) of x [B, S, H] (cdx_qkv_cache_fwd): the projection, QK norm and
+    RoPE at positions past .. past + S - 1, and the cache with the new rows appended
+    (k, v [B, nkv, past + S, hd]).  For a few queries whose keys are all cached the kernel
+    runs the causal attention too and q is None; otherwise attention is None and q is
+    [B, nq, S, hd].  past: contiguous (k, v) of [B, nkv, past, hd], or None."""
+    nat.require_device(x, mu, w_x, w_mu, q_norm_w, k_norm_w, *(past or ()), what="qkv_cache")
+    B, S, _ = x.shape
+    x2, ldx = _rows_view(x, H)
+    if ldx == 0:
+        x2, ldx = x.contiguous(), H
+    mu2, ldmu = None, 0
+    if mu is not None:
+        mu2, ldmu = _rows_view(mu.expand(B, S, H) if mu.shape[:-1] != (B, S) else mu, H)
+    wx_ptr, wmu_ptr, ldw = _weight_sources(w_x, w_mu, mu2, H, "qkv_cache")
+    if q_norm_w is not None:
+        q_norm_w = q_norm_w.to(x.dtype).contiguous()
+        k_norm_w = k_norm_w.to(x.dtype).contiguous()
+    pk, pv = past if past is not None else (None, None)
+    P = pk.shape[2] if past is not None else 0
+    attend = S <= _ATTEND_ROWS and P >= S
+    new = lambda *shape: torch.empty(shape, dtype=x.dtype, device=x.device)  # noqa: E731
+    q = None if attend else new(B, nq, S, hd)
+    attn = new(B, S, nq * hd) if attend else None
+    k, v = new(B, nkv, P + S, hd), new(B, nkv, P + S, hd)
+    lib = nat.lib()
+    ws = lib.cdx_qkv_cache_workspace_bytes(B, S, nq, nkv, hd)
+    work = torch.empty(ws, dtype=torch.uint8, device=x.device)
+    with nat.launch_region("mu_qkv", x.device, M=B * S, H=H, N=(nq + 2 * nkv) * hd, mu=mu is not None):
+        nat.check(lib.cdx_qkv_cache_fwd(
+            x2.data_ptr(), ldx, nat.ptr(mu2), ldmu, wx_ptr, wmu_ptr, ldw, B, S, H, nq, nkv, hd, nat.ptr(q_norm_w),
+            nat.ptr(k_norm_w), float(eps), cos_sin.data_ptr(), cos_sin.shape[0], nat.ptr(pk), nat.ptr(pv), P,
+            nat.ptr(q), k.data_ptr(), v.data_ptr(), nat.ptr(attn), hd ** -0.5, work.data_ptr(), ws,
+            nat.stream_of(x)), "cdx_qkv_cache_fwd")
+    return q, attn, k, v
+
+
+def cache_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+    """softmax(q k^T / sqrt(D), top-left causal) v merged to [B, S, nq * D], for q
+    [B, nq, S, D] and a cache k, v [B, nkv, rows >= S, D] (contiguous, D a multiple of 8 up
+    to 128): only the first S keys are visible to any query and read
+    (cdx_vt_pack, cdx_attention_cache_fwd)."""
+    nat.require_device(q, k, v, what="cache_attention")
+    B, nq, S, D = q.shape
+    nkv, rows = k.shape[1], k.shape[2]
+    if k.shape != (B, nkv, rows, D) or v.shape != k.shape or rows < S:
+        raise ValueError("cache_attention: q/k/v shapes do not match")
+    if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
+        raise ValueError("cache_attention: q, k and v must be contiguous")
+    vt_ld = vt_ld_for(S)
+    vt = torch.empty(B, nkv, D, vt_ld, dtype=q.dtype, device=q.device)
+    out = torch.empty(B, S, nq * D, dtype=q.dtype, device=q.device)
+    lib, stream = nat.lib(), nat.stream_of(q)
+    with nat.launch_region("attention", q.device, B=B, S=S, nq=nq, D=D):
+        nat.check(lib.cdx_vt_pack(v.data_ptr(), B * nkv, rows, S, D, vt.data_ptr(), vt_ld, stream), "cdx_vt_pack")
+        nat.check(lib.cdx_attention_cache_fwd(q.data_ptr(), k.data_ptr(), vt.data_ptr(), B, S, rows, nq, nkv, D, vt_ld,
+                                              D ** -0.5, out.data_ptr(), stream), "cdx_attention_cache_fwd")
+    return out
+
+
 def fused_mu_qkv_projection(x: torch.Tensor, mu: Optional[torch.Tensor], wq: torch.Tensor,
                             wk: torch.Tensor, wv: torch.Tensor, mu_wq: torch.Tensor,
                             mu_wk: torch.Tensor, mu_wv: torch.Tensor
@@ -277,6 +350,19 @@ class FusedMuQKVProjection(nn.Module):
         out = mu_qkv_project(x, mu, w_x, self.hidden_size, w_mu=w_mu)
         return (out[..., : self.q_dim], out[..., self.q_dim: self.q_dim + self.kv_dim],
                 out[..., self.q_dim + self.kv_dim:])
+
+
+def _plain_norm(m: nn.Module, D: int) -> bool:
+    """Whether m is an unhooked nn.RMSNorm over D values with a weight and an eps."""
+    return (type(m) is nn.RMSNorm and m.weight is not None and m.weight.shape == (D,) and m.eps is not None
+            and not (m._forward_hooks or m._forward_pre_hooks))
+
+
+def _plain_linear(m: nn.Module) -> bool:
+    """Whether calling m is exactly F.linear(x, m.weight): no subclass, bias, hook or autocast."""
+    return (type(m) is nn.Linear and m.bias is None and type(m.weight) is nn.Parameter
+            and not (m._forward_hooks or m._forward_pre_hooks or torch.is_autocast_enabled()
+                     or nn.modules.module._has_any_global_hook()))
 
 
 class QKVWeights:
@@ -380,16 +466,72 @@ class ComplexityAttention(nn.Module):
         handles head dims 32, 64 and 128 and H a multiple of 64)."""
         return self.head_dim in (32, 64, 128) and self.hidden_size % 64 == 0
 
+    @property
+    def other_head_dim(self) -> bool:
+        """Whether the heads run on the kernels through cdx_qkv_cache_fwd alone: a head dim
+        that is a multiple of 8 up to 128 other than 32, 64 and 128, with the module's own
+        norms and rotary tables in place."""
+        D = self.head_dim
+        return (D not in (32, 64, 128) and D % 8 == 0 and D <= 128 and self.hidden_size % 64 == 0
+                and type(self.rotary_emb) is RotaryEmbedding
+                and (not self.use_qk_norm or (_plain_norm(self.q_norm, D) and _plain_norm(self.k_norm, D)
+                                              and self.q_norm.eps == self.k_norm.eps)))
+
+    def _cache_fits(self, past, x: torch.Tensor) -> bool:
+        """Whether the kernels take this KV cache (None does): plain contiguous tensors of the
+        module's shape.  Any other goes through torch.cat and SDPA."""
+        if past is None:
+            return True
+        k, v = past
+        B, S, _ = x.shape
+        return (k.dim() == 4 and k.shape == (B, self.num_kv_heads, k.shape[2], self.head_dim) and v.shape == k.shape
+                and k.shape[2] > 0 and 2 * B * self.num_kv_heads * (k.shape[2] + S) * self.head_dim // 8 < 2 ** 31
+                and all(t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
+                        and not (t.requires_grad and torch.is_grad_enabled()) for t in (k, v)))
+
+    def _cache_attention(self, x: torch.Tensor, mu: Optional[torch.Tensor], past, use_cache: bool,
+                         residual: Optional[torch.Tensor]):
+        """The attention (no mask, no dropout) with a KV cache, of a few rows or at another
+        head dim, on the kernels."""
+        nat.require_device(x, what="ComplexityAttention")
+        B, S, _ = x.shape
+        H, D, nq, nkv = self.hidden_size, self.head_dim, self.num_heads, self.num_kv_heads
+        past_len = past[0].shape[2] if past is not None else 0
+        w_x, w_mu = self.qkv_weights()
+        table = self.rotary_emb.cos_sin_table(past_len + S, x.device)
+        qn = (self.q_norm.weight, self.k_norm.weight) if self.use_qk_norm else (None, None)
+        eps = self.q_norm.eps if self.use_qk_norm else 0.0
+        if D not in (32, 64, 128) or few_rows(B * S, (nq + 2 * nkv) * D):
+            # A few rows: the fused epilogue needs whole heads in a tile, i.e. a handful of
+            # blocks (one 1B layer, 4 rows: 78 us on 16 CUs; product and pass here 17 us).
+            q, attn, k, v = qkv_cache(x, mu, w_x, w_mu, H, nq, nkv, D, *qn, eps, table, past)
+            if attn is None:
+                attn = cache_attention(q, k, v)
+        else:
+            q, k, v = mu_qkv_rope(x, mu, w_x, H, nq, nkv, D, *qn, eps, table, past_len, w_mu=w_mu)
+            if past is not None:
+                k, v = torch.cat([past[0], k], dim=2), torch.cat([past[1], v], dim=2)
+            attn = cache_attention(q, k, v)
+        return self._out_proj(attn, residual), (k, v) if use_cache else None
+
     def _out_proj(self, attn: torch.Tensor, residual: Optional[torch.Tensor]) -> torch.Tensor:
         """o_proj(attn), or with ``residual``: residual + o_proj(attn) written into residual
         (one GEMM with beta = 1, the block's residual add of core/layer.py:174).  o_proj is
         not one of the path's three pieces; hipBLASLt's beta = 1 GEMM ran the 1B forward
         0.8% faster than the tile engine's o_proj + residual kernel (linear_residual_), so
-        the model keeps it."""
+        the model keeps it.  The few rows of a generation step run on the kernels for few
+        rows instead (4 x 2048 x 2048: 4.4 us, the library's 8.4 us), unless o_proj is
+        more than a plain Linear."""
+        w = self.o_proj.weight
+        own = (few_rows(attn.shape[0] * attn.shape[1], w.shape[0]) and _plain_linear(self.o_proj)
+               and w.dtype == attn.dtype and w.is_contiguous() and w.data_ptr() % 16 == 0
+               and w.shape[0] % 8 == 0 and w.shape[1] % 64 == 0)
         if residual is None:
-            return self.o_proj(attn)
+            return linear(attn, w) if own else self.o_proj(attn)
         if residual.shape[:-1] != attn.shape[:-1] or not residual.is_contiguous():
             raise ValueError("ComplexityAttention: residual must be contiguous and match the input rows")
+        if own and residual.dtype == attn.dtype and residual.data_ptr() % 16 == 0:
+            return linear_accumulate_(attn, w, residual)
         residual.view(-1, residual.shape[-1]).addmm_(attn.reshape(-1, attn.shape[-1]), self.o_proj.weight.t())
         return residual
 
@@ -403,18 +545,22 @@ class ComplexityAttention(nn.Module):
         B, S, _ = hidden_states.shape
         D = self.head_dim
         past_len = past_key_value[0].shape[2] if past_key_value is not None else 0
-        if self.fused_prologue and attention_mask is None and past_key_value is None and not use_cache \
-                and not (self.training and self.attention_dropout > 0):
-            # Whole attention on the kernels: fused projection (V written transposed) and
-            # the causal GQA kernel, whose output is already merged over heads.
-            w_x, w_mu = self.qkv_weights()
-            table = self.rotary_emb.cos_sin_table(S, hidden_states.device)
-            qn = (self.q_norm.weight, self.k_norm.weight) if self.use_qk_norm else (None, None)
-            eps = self.q_norm.eps if self.use_qk_norm else 0.0
-            q, k, vt = mu_qkv_rope(hidden_states, mu_prev, w_x, self.hidden_size, self.num_heads,
-                                   self.num_kv_heads, D, qn[0], qn[1], eps, table, 0, v_transposed=True,
-                                   w_mu=w_mu)
-            return self._out_proj(causal_attention(q, k, vt), residual), None
+        if attention_mask is None and not (self.training and self.attention_dropout > 0):
+            cached = past_key_value is not None or use_cache
+            fused = self.fused_prologue
+            if fused and not cached and not few_rows(B * S, (self.num_heads + 2 * self.num_kv_heads) * D):
+                # Fused projection (V written transposed) and the causal GQA kernel, whose
+                # output is already merged over heads.
+                w_x, w_mu = self.qkv_weights()
+                table = self.rotary_emb.cos_sin_table(S, hidden_states.device)
+                qn = (self.q_norm.weight, self.k_norm.weight) if self.use_qk_norm else (None, None)
+                eps = self.q_norm.eps if self.use_qk_norm else 0.0
+                q, k, vt = mu_qkv_rope(hidden_states, mu_prev, w_x, self.hidden_size, self.num_heads,
+                                       self.num_kv_heads, D, qn[0], qn[1], eps, table, 0, v_transposed=True,
+                                       w_mu=w_mu)
+                return self._out_proj(causal_attention(q, k, vt), residual), None
+            if B * S > 0 and (fused or self.other_head_dim) and self._cache_fits(past_key_value, hidden_states):
+                return self._cache_attention(hidden_states, mu_prev, past_key_value, use_cache, residual)
         if self.fused_prologue:
             # Projection, head split, QK RMSNorm and RoPE in one kernel (attention.py:120-155).
             w_x, w_mu = self.qkv_weights()

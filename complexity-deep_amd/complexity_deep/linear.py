@@ -11,7 +11,7 @@ MFMA tile engine (cdx_linear_fwd; fp32 accumulation, one bf16 rounding).
 the rounding of a separate bf16 add (cdx_linear_residual_fwd): the attention block's
 o_proj and residual add (core/attention.py:71,181, core/layer.py:174) as an operator;
 ComplexityModel keeps hipBLASLt's GEMM with beta = 1 for it, which ran the 1B forward
-0.8% faster.
+0.8% faster, except for the few rows of a generation step (``linear_accumulate_``).
 """
 
 from __future__ import annotations
@@ -83,4 +83,28 @@ def linear_residual_(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor) -
         nat.check(nat.lib().cdx_linear_residual_fwd(x2.data_ptr(), K, w.data_ptr(), K, M, K, N,
                                                     residual.data_ptr(), N, nat.stream_of(x)),
                   "cdx_linear_residual_fwd")
+    return residual
+
+
+def few_rows(M: int, N: int) -> bool:
+    """Whether a product of M rows and N output columns runs on the kernels for few rows
+    (never above 64 rows: asked of the library below that only)."""
+    return M <= 64 and nat.lib().cdx_few_rows(M, N) != 0
+
+
+def linear_accumulate_(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
+    """residual += x @ w^T in place with one rounding (a GEMM with beta = 1), for the shapes
+    of few_rows.  x [..., K], w [N, K] and residual [..., N] contiguous; K % 64 == 0,
+    N % 8 == 0."""
+    nat.require_device(x, w, residual, what="linear_accumulate_")
+    N, K = w.shape
+    if x.shape[-1] != K or residual.shape != x.shape[:-1] + (N,):
+        raise ValueError(f"linear_accumulate_: x {tuple(x.shape)}, w {tuple(w.shape)} and residual "
+                         f"{tuple(residual.shape)} do not match")
+    if not (x.is_contiguous() and w.is_contiguous() and residual.is_contiguous()):
+        raise ValueError("linear_accumulate_: contiguous tensors expected")
+    M = x.numel() // K
+    with nat.launch_region("o_proj", x.device, M=M, K=K, N=N):
+        nat.check(nat.lib().cdx_linear_accum_fwd(x.data_ptr(), K, w.data_ptr(), K, M, K, N, residual.data_ptr(), N,
+                                                 nat.stream_of(x)), "cdx_linear_accum_fwd")
     return residual

@@ -42,12 +42,14 @@ namespace {
 
 struct AttnParams {
   const uint16_t* q;   // [B, nq, S, HD]
-  const uint16_t* k;   // [B, nkv, S, HD]
+  const uint16_t* k;   // [B, nkv, kv_rows, HD]
   const uint16_t* vt;  // [B, nkv, HD, vt_ld], keys in vt_col order
   uint16_t* out;       // [B, S, nq * HD]
   int64_t S;
+  int64_t kv_rows;     // rows of a (batch, kv head) slice of k; keys 0 .. S - 1 are read
   int64_t vt_ld;
   int32_t B, nq, nkv;
+  int32_t D;           // head dim (GEN; else HD)
   int32_t q_tiles;
   float scale_log2;    // log2(e) * scale
 };
@@ -65,7 +67,11 @@ __device__ __forceinline__ void halves(float x, float& a, float& b) {
   b = __uint_as_float(r[1]);
 }
 
-template <int HD>
+// GEN: head dims p.D < HD that are a multiple of 8 (heads of 80 or 40, say) on the LDS
+// layout of HD = 64 or 128 with NKD = ceil(D / 16) contraction steps: chunks past D are
+// fetched out of range of the buffer descriptors, i.e. as zeros, in K and V^T alike, and
+// never stored.  Memory keeps rows of D values.
+template <int HD, int NKD = HD / 16, bool GEN = false>
 __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
   constexpr int KROW = HD * 2;              // bytes per K row
   constexpr int K_CPR = HD / 8;             // 16-byte chunks per K row
@@ -74,13 +80,14 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
   constexpr int V_ROWB = kAttnBN * 2;       // 128 bytes per V^T row (64 keys)
   constexpr int V_BYTES = HD * V_ROWB;      // one V^T tile
   constexpr int V_BASE = 2 * K_BYTES;       // two K buffers, then two V^T buffers
-  constexpr int NKD = HD / 16;              // K16 steps over the head dim
-  constexpr int NDB = HD / 32;              // 32-row blocks of O^T
+  constexpr int NDB = (NKD + 1) / 2;        // 32-row blocks of O^T (NKD: K16 steps over the head dim)
   constexpr int KPW = K_BYTES / 1024 / 4;   // K DMA instructions per wave and tile
   constexpr int VPW = V_BYTES / 1024 / 4;   // V^T DMA instructions per wave and tile
   constexpr int K_ROWS_DMA = 1024 / KROW;   // K rows one DMA instruction fills
   static_assert(HD == 32 || HD == 64 || HD == 128, "head dim must be 32, 64 or 128");
   static_assert(KPW >= 1 && VPW >= 1, "tile too small for the DMA layout");
+  static_assert(GEN ? (HD >= 64 && NKD * 16 <= HD) : NKD * 16 == HD, "contraction steps must fit the head dim");
+  const int D = GEN ? p.D : HD;
 
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * K_BYTES + 2 * V_BYTES];
 
@@ -109,9 +116,12 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
   bf16x8 qf[NKD];
   {
     const int64_t mr = m < S ? m : S - 1;
-    const uint16_t* qrow = p.q + (((int64_t)b * p.nq + h) * S + mr) * HD + 8 * hi;
+    const uint16_t* qrow = p.q + (((int64_t)b * p.nq + h) * S + mr) * D + 8 * hi;
 #pragma unroll
-    for (int k = 0; k < NKD; ++k) qf[k] = *reinterpret_cast<const bf16x8*>(qrow + 16 * k);
+    for (int k = 0; k < NKD; ++k) {
+      qf[k] = bf16x8{};
+      if (!GEN || 16 * k + 8 * hi < D) qf[k] = *reinterpret_cast<const bf16x8*>(qrow + 16 * k);
+    }
   }
 
   // ---- DMA sources ---------------------------------------------------------------
@@ -125,21 +135,24 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
   // move along a row by their key position (scalar offset): columns up to vt_ld are
   // inside the slice and finite by contract.
   const __amdgpu_buffer_rsrc_t rs_k =
-      make_rsrc(p.k + ((int64_t)b * p.nkv + kvh) * S * HD, (uint32_t)(S * HD * 2));
-  const __amdgpu_buffer_rsrc_t rs_v = make_rsrc(p.vt + ((int64_t)b * p.nkv + kvh) * HD * p.vt_ld);
+      make_rsrc(p.k + ((int64_t)b * p.nkv + kvh) * p.kv_rows * D, (uint32_t)(S * D * 2));
+  const __amdgpu_buffer_rsrc_t rs_v = make_rsrc(p.vt + ((int64_t)b * p.nkv + kvh) * D * p.vt_ld,
+                                                GEN ? (uint32_t)(D * p.vt_ld * 2) : 0xFFFFFFFFu);
+  constexpr uint32_t kOutside = 0x80000000u;  // (GEN: the host keeps K and V^T slices below 2 GB)
   uint32_t k_off[KPW], v_off[VPW];
 #pragma unroll
   for (int j = 0; j < KPW; ++j) {
     const int r = (wave * KPW + j) * K_ROWS_DMA + lane / K_CPR;
-    k_off[j] = (uint32_t)(r * HD + ((lane % K_CPR) ^ ((r / K_RPL) % K_CPR)) * 8) * 2;
+    const int c = ((lane % K_CPR) ^ ((r / K_RPL) % K_CPR)) * 8;
+    k_off[j] = GEN && c >= D ? kOutside : (uint32_t)(r * D + c) * 2;
   }
 #pragma unroll
   for (int j = 0; j < VPW; ++j) {
     const int d = (wave * VPW + j) * 8 + lane / 8;
-    v_off[j] = (uint32_t)((int64_t)d * p.vt_ld + ((lane % 8) ^ ((d / 2) % 8)) * 8) * 2;
+    v_off[j] = GEN && d >= D ? kOutside : (uint32_t)((int64_t)d * p.vt_ld + ((lane % 8) ^ ((d / 2) % 8)) * 8) * 2;
   }
   auto issue_k = [&](int t, int buf) __attribute__((always_inline)) {
-    const uint32_t tile_off = (uint32_t)t * (kAttnBN * HD * 2);
+    const uint32_t tile_off = (uint32_t)t * (kAttnBN * 2) * (uint32_t)D;
 #pragma unroll
     for (int j = 0; j < KPW; ++j)
       buf_dma16(rs_k, k_off[j] + tile_off, 0u, lds + buf * K_BYTES + (wave * KPW + j) * 1024);
@@ -385,22 +398,77 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnParams p) {
   // The wave's own LDS writes complete before its reads (and stay ahead of them).
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
   const int jc = lane % OCH;
-  uint16_t* obase = p.out + (int64_t)h * HD + jc * 8;
+  if (GEN && jc * 8 >= D) return;
+  uint16_t* obase = p.out + (int64_t)h * D + jc * 8;
 #pragma unroll
   for (int i = 0; i < 32 / ORPI; ++i) {
     const int r = i * ORPI + lane / OCH;
     const uint4 v = *reinterpret_cast<const uint4*>(ost + r * OROWB + ((jc ^ (r % OCH)) << 4));
     const int64_t mr = mw + r;
-    if (mr < S) *reinterpret_cast<uint4*>(obase + ((int64_t)b * S + mr) * ((int64_t)p.nq * HD)) = v;
+    if (mr < S) *reinterpret_cast<uint4*>(obase + ((int64_t)b * S + mr) * ((int64_t)p.nq * D)) = v;
   }
 }
 
-template <int HD>
-int launch_attn(const AttnParams& p, hipStream_t s) {
+template <int HD, int NKD = HD / 16, bool GEN = false>
+int launch_attn(const AttnParams& p, hipStream_t s, const char* name) {
   const int64_t blocks = (int64_t)p.q_tiles * p.B * p.nq;
-  if (blocks > INT32_MAX) return fail(CDX_EUNSUPPORTED, "cdx_attention_fwd: problem too large");
-  attn_fwd_kernel<HD><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(p);
-  return check_launch("cdx_attention_fwd");
+  if (blocks > INT32_MAX) return fail(CDX_EUNSUPPORTED, "%s: problem too large", name);
+  attn_fwd_kernel<HD, NKD, GEN><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(p);
+  return check_launch(name);
+}
+
+int attention(const char* name, const uint16_t* q, const uint16_t* k, const uint16_t* vt, int64_t B, int64_t S,
+              int64_t kv_rows, int32_t nq, int32_t nkv, int32_t hd, int64_t vt_ld, float scale, uint16_t* out,
+              void* stream) {
+  const bool gen = hd != 32 && hd != 64 && hd != 128;
+  if (B < 0 || S < 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || kv_rows < S)
+    return fail(CDX_EINVAL, "%s: bad shape B=%lld S=%lld nq=%d nkv=%d", name, (long long)B, (long long)S, nq, nkv);
+  if (vt_ld < S || vt_ld % 64 != 0)
+    return fail(CDX_EINVAL, "%s: vt_ld=%lld must be a multiple of 64 that is >= S", name, (long long)vt_ld);
+  if (!(scale > 0.f)) return fail(CDX_EINVAL, "%s: scale must be > 0", name);
+  if (B == 0 || S == 0) return CDX_OK;
+  if ((S + kAttnBM - 1) / kAttnBM > INT32_MAX || B * nq > INT32_MAX)
+    return fail(CDX_EUNSUPPORTED, "%s: problem too large", name);
+  // The kernel addresses one (batch, kv head) slice of K and of V^T with 32-bit offsets
+  // (31-bit ones when it masks columns past the head dim); a K tile's offsets reach up to
+  // 64 rows past the slice (those rows read as zeros).
+  const int64_t most = gen ? (int64_t)INT32_MAX : (int64_t)UINT32_MAX;
+  if ((S + 64) * hd * 2 > most || vt_ld * hd * 2 > most)
+    return fail(CDX_EUNSUPPORTED, "%s: a K or V^T head slice must fit %d GB (S=%lld)", name, gen ? 2 : 4, (long long)S);
+  if (!q || !k || !vt || !out) return fail(CDX_EINVAL, "%s: null pointer", name);
+  if (!aligned16(q) || !aligned16(k) || !aligned16(vt) || !aligned16(out))
+    return fail(CDX_EUNSUPPORTED, "%s: pointers must be 16-byte aligned", name);
+  AttnParams p{};
+  p.q = q;
+  p.k = k;
+  p.vt = vt;
+  p.out = out;
+  p.S = S;
+  p.kv_rows = kv_rows;
+  p.vt_ld = vt_ld;
+  p.B = (int32_t)B;
+  p.nq = nq;
+  p.nkv = nkv;
+  p.D = hd;
+  p.q_tiles = (int32_t)((S + kAttnBM - 1) / kAttnBM);
+  p.scale_log2 = scale * 1.4426950408889634f;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  switch (hd) {
+    case 32: return launch_attn<32>(p, s, name);
+    case 64: return launch_attn<64>(p, s, name);
+    case 128: return launch_attn<128>(p, s, name);
+    default: break;
+  }
+  switch ((hd + 15) / 16) {
+    case 1:
+    case 2: return launch_attn<64, 2, true>(p, s, name);
+    case 3: return launch_attn<64, 3, true>(p, s, name);
+    case 4: return launch_attn<64, 4, true>(p, s, name);
+    case 5: return launch_attn<128, 5, true>(p, s, name);
+    case 6: return launch_attn<128, 6, true>(p, s, name);
+    case 7: return launch_attn<128, 7, true>(p, s, name);
+    default: return launch_attn<128, 8, true>(p, s, name);
+  }
 }
 
 }  // namespace
@@ -412,39 +480,18 @@ extern "C" int cdx_attention_fwd(const uint16_t* q, const uint16_t* k, const uin
   using namespace cdx;
   clear_error();
   const char* name = "cdx_attention_fwd";
-  if (B < 0 || S < 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0)
-    return fail(CDX_EINVAL, "%s: bad shape B=%lld S=%lld nq=%d nkv=%d", name, (long long)B, (long long)S, nq, nkv);
   if (hd != 32 && hd != 64 && hd != 128)
     return fail(CDX_EUNSUPPORTED, "%s: head dim %d must be 32, 64 or 128", name, hd);
-  if (vt_ld < S || vt_ld % 64 != 0)
-    return fail(CDX_EINVAL, "%s: vt_ld=%lld must be a multiple of 64 that is >= S", name, (long long)vt_ld);
-  if (!(scale > 0.f)) return fail(CDX_EINVAL, "%s: scale must be > 0", name);
-  if (B == 0 || S == 0) return CDX_OK;
-  if ((S + kAttnBM - 1) / kAttnBM > INT32_MAX || B * nq > INT32_MAX)
-    return fail(CDX_EUNSUPPORTED, "%s: problem too large", name);
-  // The kernel addresses one (batch, kv head) slice of K and of V^T with 32-bit offsets;
-  // a K tile's offsets reach up to 64 rows past the slice (those rows read as zeros).
-  if ((S + 64) * hd * 2 > (int64_t)UINT32_MAX || vt_ld * hd * 2 > (int64_t)UINT32_MAX)
-    return fail(CDX_EUNSUPPORTED, "%s: a K or V^T head slice must fit 4 GB (S=%lld)", name, (long long)S);
-  if (!q || !k || !vt || !out) return fail(CDX_EINVAL, "%s: null pointer", name);
-  if (!aligned16(q) || !aligned16(k) || !aligned16(vt) || !aligned16(out))
-    return fail(CDX_EUNSUPPORTED, "%s: pointers must be 16-byte aligned", name);
-  AttnParams p{};
-  p.q = q;
-  p.k = k;
-  p.vt = vt;
-  p.out = out;
-  p.S = S;
-  p.vt_ld = vt_ld;
-  p.B = (int32_t)B;
-  p.nq = nq;
-  p.nkv = nkv;
-  p.q_tiles = (int32_t)((S + kAttnBM - 1) / kAttnBM);
-  p.scale_log2 = scale * 1.4426950408889634f;
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  switch (hd) {
-    case 32: return launch_attn<32>(p, s);
-    case 64: return launch_attn<64>(p, s);
-    default: return launch_attn<128>(p, s);
-  }
+  return attention(name, q, k, vt, B, S, S, nq, nkv, hd, vt_ld, scale, out, stream);
+}
+
+extern "C" int cdx_attention_cache_fwd(const uint16_t* q, const uint16_t* k, const uint16_t* vt, int64_t B, int64_t S,
+                                       int64_t kv_rows, int32_t nq, int32_t nkv, int32_t hd, int64_t vt_ld,
+                                       float scale, uint16_t* out, void* stream) {
+  using namespace cdx;
+  clear_error();
+  const char* name = "cdx_attention_cache_fwd";
+  if (hd <= 0 || hd > 128 || hd % 8 != 0)
+    return fail(CDX_EUNSUPPORTED, "%s: head dim %d must be a multiple of 8 and <= 128", name, hd);
+  return attention(name, q, k, vt, B, S, kv_rows, nq, nkv, hd, vt_ld, scale, out, stream);
 }

@@ -599,11 +599,14 @@ extern "C" int cdx_linear_fwd(const uint16_t* x, int64_t ldx, const uint16_t* w,
   return launch<ALoad::kDense, Epi::kStore>(p, reinterpret_cast<hipStream_t>(stream), name);
 }
 
-extern "C" int cdx_linear_residual_fwd(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, int64_t M,
-                                       int32_t K, int32_t N, uint16_t* residual, int64_t ldr, void* stream) {
-  using namespace cdx;
+namespace cdx {
+namespace {
+
+// residual += x @ w^T.  single: one rounding of the fp32 sum, for products of a few rows
+// (skinny_fits); else the rounded product, then a bf16 add.
+int linear_residual(const char* name, const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, int64_t M,
+                    int32_t K, int32_t N, uint16_t* residual, int64_t ldr, bool single, void* stream) {
   clear_error();
-  const char* name = "cdx_linear_residual_fwd";
   if (M < 0 || K <= 0 || N <= 0) return fail(CDX_EINVAL, "%s: bad shape M=%lld K=%d N=%d", name, (long long)M, K, N);
   if (K % 64 != 0) return fail(CDX_EUNSUPPORTED, "%s: K=%d must be a multiple of 64", name, K);
   // The residual is read and written in whole 16-byte pieces.
@@ -617,8 +620,9 @@ extern "C" int cdx_linear_residual_fwd(const uint16_t* x, int64_t ldx, const uin
   if (!aligned16(x) || !aligned16(w) || !aligned16(residual))
     return fail(CDX_EUNSUPPORTED, "%s: pointers must be 16-byte aligned", name);
   if (skinny_fits(M, N))
-    return skinny_gemm(skinny_params(x, ldx, w, ldw, M, K, N, residual, ldr), SkinnyEpi::kResid,
-                       reinterpret_cast<hipStream_t>(stream), name);
+    return skinny_gemm(skinny_params(x, ldx, w, ldw, M, K, N, residual, ldr),
+                       single ? SkinnyEpi::kAccum : SkinnyEpi::kResid, reinterpret_cast<hipStream_t>(stream), name);
+  if (single) return fail(CDX_EUNSUPPORTED, "%s: M=%lld has too many rows", name, (long long)M);
   GemmParams p{};
   p.a = x;
   p.lda = ldx;
@@ -634,4 +638,17 @@ extern "C" int cdx_linear_residual_fwd(const uint16_t* x, int64_t ldx, const uin
   p.ldc = ldr;
   p.mt_count = (int32_t)cdiv(M, kBM);
   return launch<ALoad::kDense, Epi::kScatterAdd>(p, reinterpret_cast<hipStream_t>(stream), name);
+}
+
+}  // namespace
+}  // namespace cdx
+
+extern "C" int cdx_linear_residual_fwd(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, int64_t M,
+                                       int32_t K, int32_t N, uint16_t* residual, int64_t ldr, void* stream) {
+  return cdx::linear_residual("cdx_linear_residual_fwd", x, ldx, w, ldw, M, K, N, residual, ldr, false, stream);
+}
+
+extern "C" int cdx_linear_accum_fwd(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, int64_t M,
+                                    int32_t K, int32_t N, uint16_t* residual, int64_t ldr, void* stream) {
+  return cdx::linear_residual("cdx_linear_accum_fwd", x, ldx, w, ldw, M, K, N, residual, ldr, true, stream);
 }

@@ -16,8 +16,9 @@ constexpr int kSkinnyRows = 64;
 // 64 rows, 4096 columns (K = 4096) 21.3 / 28.3, 8192 columns 21.5 / 17.1).
 bool skinny_fits(int64_t M, int64_t N);
 
-// kResid adds the rounded product to C (the rounding of a separate bf16 add).
-enum class SkinnyEpi { kStore, kBiasClamp, kResid };
+// kF32 stores the fp32 sums; kResid adds the rounded product to bf16 C (the rounding of a
+// separate bf16 add); kAccum adds the fp32 product to bf16 C with one rounding.
+enum class SkinnyEpi { kStore, kF32, kBiasClamp, kResid, kAccum };
 
 struct SkinnyParams {
   const uint16_t* a;   // [M][lda], K columns [0, k_split)
@@ -29,7 +30,7 @@ struct SkinnyParams {
   int64_t ldb;
   int32_t k_split;     // == K without a second source; a multiple of 64
   int32_t M, N, K;     // K a multiple of 64
-  uint16_t* c;         // row stride ldc; columns up to round_up(N, 8) are written
+  void* c;             // bf16 (fp32 for kF32), row stride ldc; columns up to round_up(N, 8) are written
   int64_t ldc;
   const uint16_t* bias;  // kBiasClamp: c = clamp(acc + clamp(bias[n], bias_lo, bias_hi), lo, hi)
   float bias_lo, bias_hi, lo, hi;

@@ -145,6 +145,10 @@ __global__ __launch_bounds__(64 * W) void skinny_kernel(const SkinnyParams p) {
     if (m >= p.M || n >= ((p.N + 7) & ~7)) continue;
     const f32x4 t = it.template total<NB * MT, W>(red, blk);
     float y[4] = {t[0], t[1], t[2], t[3]};
+    if constexpr (EPI == SkinnyEpi::kF32) {
+      *reinterpret_cast<float4*>(static_cast<float*>(p.c) + (int64_t)m * p.ldc + n) = make_float4(y[0], y[1], y[2], y[3]);
+      continue;
+    }
     if constexpr (EPI == SkinnyEpi::kBiasClamp) {
       const uint2 bw = *reinterpret_cast<const uint2*>(p.bias + n);
       const float bb[4] = {__uint_as_float(bw.x << 16), __uint_as_float(bw.x & 0xffff0000u),
@@ -155,13 +159,14 @@ __global__ __launch_bounds__(64 * W) void skinny_kernel(const SkinnyParams p) {
         y[j] = fminf(fmaxf(v, p.lo), p.hi);
       }
     }
-    uint2* dst = reinterpret_cast<uint2*>(p.c + (int64_t)m * p.ldc + n);
-    if constexpr (EPI == SkinnyEpi::kResid) {
+    uint2* dst = reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.c) + (int64_t)m * p.ldc + n);
+    if constexpr (EPI == SkinnyEpi::kResid || EPI == SkinnyEpi::kAccum) {
       const uint2 cw = *dst;
       const float old[4] = {__uint_as_float(cw.x << 16), __uint_as_float(cw.x & 0xffff0000u),
                             __uint_as_float(cw.y << 16), __uint_as_float(cw.y & 0xffff0000u)};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) y[j] = old[j] + bf16_bits_to_f32(f32_to_bf16_bits(y[j]));
+      for (int j = 0; j < 4; ++j)
+        y[j] = old[j] + (EPI == SkinnyEpi::kResid ? bf16_bits_to_f32(f32_to_bf16_bits(y[j])) : y[j]);
     }
     *dst = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
   }
@@ -176,7 +181,9 @@ int launch_skinny(const SkinnyParams& p, SkinnyEpi epi, hipStream_t s, const cha
     case SkinnyEpi::kBiasClamp:
       skinny_kernel<MT, NB, W, CH, HALF, SkinnyEpi::kBiasClamp><<<grid, block, 0, s>>>(p);
       break;
-    default: skinny_kernel<MT, NB, W, CH, HALF, SkinnyEpi::kResid><<<grid, block, 0, s>>>(p); break;
+    case SkinnyEpi::kF32: skinny_kernel<MT, NB, W, CH, HALF, SkinnyEpi::kF32><<<grid, block, 0, s>>>(p); break;
+    case SkinnyEpi::kResid: skinny_kernel<MT, NB, W, CH, HALF, SkinnyEpi::kResid><<<grid, block, 0, s>>>(p); break;
+    default: skinny_kernel<MT, NB, W, CH, HALF, SkinnyEpi::kAccum><<<grid, block, 0, s>>>(p); break;
   }
   return check_launch(name);
 }

@@ -320,6 +320,46 @@ int cdx_mu_qkv_rope_bcast_fwd(const uint16_t* x_dev, int64_t ldx, const uint16_t
                               void* stream);
 
 /*
+ * 1 if a product of M rows and N output columns runs on the kernels for few rows (a
+ * generation step: M <= 64, and fewer the wider the output), 0 otherwise.
+ */
+int32_t cdx_few_rows(int64_t M, int64_t N);
+
+/*
+ * mu-QKV projection, QK norm, RoPE and the KV cache of a call with S new tokens per
+ * sequence after `past` cached ones (two launches):
+ *   [q | k | v] = [x | mu] @ [w_x | w_mu]^T        (as cdx_mu_qkv_fwd)
+ *   q, k normalised and rotated as in cdx_mu_qkv_rope_fwd at positions past + s
+ *   k_out, v_out [B, nkv, past + S, hd] = past_k, past_v [B, nkv, past, hd], then the new rows
+ * and either q_out [B, nq, S, hd], or with attn_out (q_out NULL; S <= 16 and past >= S) the
+ * attention itself, [B, S, nq * hd]: the causal mask is aligned at the top left (query s
+ * sees keys 0 .. s of the whole cache), so every key lies among the cached ones.
+ * hd: any multiple of 8 up to 128.  For cdx_few_rows shapes the projection reaches the norm
+ * in fp32; for larger ones it is rounded to bf16 once before (heads of 32, 64 and 128 have
+ * cdx_mu_qkv_rope_fwd for those).
+ *   work  device scratch of cdx_qkv_cache_workspace_bytes, written on every call.
+ *
+ * Replaces: core/attention.py:120-175 (projection, norms, rotary, torch.cat with the cache,
+ * and for a step repeat_interleave and scaled_dot_product_attention).
+ */
+size_t cdx_qkv_cache_workspace_bytes(int64_t B, int64_t S, int32_t nq, int32_t nkv, int32_t hd);
+int cdx_qkv_cache_fwd(const uint16_t* x_dev, int64_t ldx, const uint16_t* mu_dev, int64_t ldmu,
+                      const uint16_t* w_x_dev, const uint16_t* w_mu_dev, int64_t ldw, int64_t B, int64_t S, int32_t H,
+                      int32_t nq, int32_t nkv, int32_t hd, const uint16_t* q_norm_w_dev,
+                      const uint16_t* k_norm_w_dev, float eps, const float* cos_sin_dev, int64_t n_pos,
+                      const uint16_t* past_k_dev, const uint16_t* past_v_dev, int64_t past, uint16_t* q_out_dev,
+                      uint16_t* k_out_dev, uint16_t* v_out_dev, uint16_t* attn_out_dev, float scale, void* work_dev,
+                      size_t work_bytes, void* stream);
+
+/*
+ * The first S rows of each of `slabs` matrices v [rows][hd] in the transposed layout of
+ * cdx_attention_fwd, vt [slabs][hd][vt_ld] (columns of tokens >= S up to the next multiple
+ * of 64 are cleared).  hd: a multiple of 8 up to 128.
+ */
+int cdx_vt_pack(const uint16_t* v_dev, int64_t slabs, int64_t rows, int64_t S, int32_t hd, uint16_t* vt_dev,
+                int64_t vt_ld, void* stream);
+
+/*
  * mu guidance, the producer of the next layer's mu operand:
  *   out[t, n] = clamp(sum_k h[t, k] w[n, k] + clamp(mu[n], mu_lo, mu_hi), lo, hi)
  * h [T, H] bf16, w [H, H] bf16 (nn.Linear layout, [out, in]), mu [H] bf16 (the
@@ -354,6 +394,15 @@ int cdx_mu_guidance_fwd(const uint16_t* h_dev, int64_t T, int32_t H, const uint1
 int cdx_attention_fwd(const uint16_t* q_dev, const uint16_t* k_dev, const uint16_t* vt_dev, int64_t B,
                       int64_t S, int32_t nq, int32_t nkv, int32_t hd, int64_t vt_ld, float scale,
                       uint16_t* out_dev, void* stream);
+
+/*
+ * cdx_attention_fwd for S queries over the first S keys of a cache whose slices hold
+ * kv_rows >= S rows (k [B, nkv, kv_rows, hd]; vt from cdx_vt_pack over the same rows), at
+ * any head dim that is a multiple of 8 up to 128.
+ */
+int cdx_attention_cache_fwd(const uint16_t* q_dev, const uint16_t* k_dev, const uint16_t* vt_dev, int64_t B,
+                            int64_t S, int64_t kv_rows, int32_t nq, int32_t nkv, int32_t hd, int64_t vt_ld,
+                            float scale, uint16_t* out_dev, void* stream);
 
 /* ---- expert map (host) ---------------------------------------------------- */
 
@@ -408,6 +457,13 @@ int cdx_linear_fwd(const uint16_t* x_dev, int64_t ldx, const uint16_t* w_dev, in
  */
 int cdx_linear_residual_fwd(const uint16_t* x_dev, int64_t ldx, const uint16_t* w_dev, int64_t ldw, int64_t M,
                             int32_t K, int32_t N, uint16_t* residual_dev, int64_t ldr, void* stream);
+
+/*
+ * residual[M, N] = bf16(residual + x[M, K] @ w[N, K]^T), in place, with one rounding (a GEMM
+ * with beta = 1), for cdx_few_rows shapes only; otherwise as cdx_linear_residual_fwd.
+ */
+int cdx_linear_accum_fwd(const uint16_t* x_dev, int64_t ldx, const uint16_t* w_dev, int64_t ldw, int64_t M,
+                         int32_t K, int32_t N, uint16_t* residual_dev, int64_t ldr, void* stream);
 
 /* ---- measurement ---------------------------------------------------------- */
 
