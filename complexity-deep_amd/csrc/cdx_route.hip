@@ -22,8 +22,10 @@
 // The count table is the only scratch: caller workspace (cdx_route_plan) or a
 // library-owned device array (cdx_route_plan_noalloc).  Nothing needs zeroing: the
 // count launch writes every entry the scatter launch reads.
+// Up to kOneBlockTokens tokens a plan is one block and one launch (route_one_kernel): all
+// ballots first, their counts in LDS, one scan, then the positions.
 // cdx_route_plans runs L plans over the same ids, one per expert map (a model's
-// layers each route through their own map), in the same two launches: the plan
+// layers each route through their own map), in the same launches: the plan
 // index is blockIdx.y, and every output and the count table gain a leading [L] axis.
 #include <mutex>
 
@@ -202,6 +204,91 @@ __global__ __launch_bounds__(256) void route_scatter_kernel(const int32_t* __res
   }
 }
 
+// The whole plan of T <= kOneBlockTokens tokens in one block (plan blockIdx.y through
+// maps.m[y]): wave w takes chunks w, w + waves, ... of 64 tokens.  A call of few tokens is
+// all latency: two launches and a count table between them took 9.2 us at 4 tokens, 9.1 at
+// 2048 and 12.2 at 4096 (8 experts), this takes 3.4, 5.3 and 9.4 (18 plans of 2048 tokens
+// 9.6 -> 5.5).  Past kOneBlockTokens one CU's lookups and scatter outgrow the second launch.
+constexpr int kOneBlockTokens = 4096;
+constexpr int kOneRounds = kOneBlockTokens / kRound;
+
+__global__ __launch_bounds__(kRound) void route_one_kernel(const int64_t* __restrict__ ids, const MapSet maps,
+                                                           int64_t V, int E, int T, int32_t* __restrict__ expert_id,
+                                                           int32_t* __restrict__ perm, int32_t* __restrict__ inv_perm,
+                                                           int32_t* __restrict__ counts,
+                                                           int32_t* __restrict__ offsets) {
+  __shared__ int cnt[kOneRounds * kChunks][kMaxE + 1];  // per chunk: counts, then start positions
+  const int64_t* map = maps.m[blockIdx.y];
+  const int64_t y = blockIdx.y;
+  expert_id += y * T;
+  perm += y * T;
+  inv_perm += y * T;
+  counts += y * E;
+  offsets += y * (E + 1);
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int chunks = (T + kWave - 1) / kWave;
+
+  int ev[kOneRounds], rank[kOneRounds];
+#pragma unroll
+  for (int j = 0; j < kOneRounds; ++j) {
+    const int t = (wave + j * waves) * kWave + lane;
+    ev[j] = -1;
+    if (t < T) {
+      ev[j] = lookup_expert(ids, map, V, E, t);
+      expert_id[t] = ev[j];
+    }
+  }
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+  for (int j = 0; j < kOneRounds; ++j) {
+    const int c = wave + j * waves;
+    rank[j] = 0;
+    if (c < chunks) {
+      for (int x = 0; x < E; ++x) {
+        const uint64_t m = __ballot(ev[j] == x);
+        if (ev[j] == x) rank[j] = __popcll(m & below);
+        if (lane == 0) cnt[c][x] = __popcll(m);
+      }
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    // Lane x scans expert x over the chunks, then the totals over the experts.
+    int run = 0;
+    if (lane < E)
+      for (int c = 0; c < chunks; ++c) run += cnt[c][lane];
+    const int total = run;
+    int incl = total;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int up = __shfl_up(incl, d);
+      incl += lane >= d ? up : 0;
+    }
+    if (lane < E) {
+      counts[lane] = total;
+      offsets[lane] = incl - total;
+      if (lane == E - 1) offsets[E] = incl;
+      int pos = incl - total;
+      for (int c = 0; c < chunks; ++c) {
+        const int n = cnt[c][lane];
+        cnt[c][lane] = pos;
+        pos += n;
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kOneRounds; ++j) {
+    const int c = wave + j * waves, t = c * kWave + lane;
+    if (t < T) {
+      const int pos = cnt[c][ev[j]] + rank[j];
+      perm[pos] = t;
+      inv_perm[t] = pos;
+    }
+  }
+}
+
 // Both launches of L <= kMaxMaps plans over the same ids (plan y through maps[y],
 // outputs at row y of each [L, ...] array); blk_counts holds L * nblk * E ints.
 int route_plan_launch(const int64_t* ids, int64_t T, const int64_t* const* maps, int32_t L, int64_t V, int32_t E,
@@ -211,6 +298,12 @@ int route_plan_launch(const int64_t* ids, int64_t T, const int64_t* const* maps,
   const int nblk = (int)((T + tpb - 1) / tpb);
   MapSet ms{};
   for (int y = 0; y < L; ++y) ms.m[y] = maps[y];
+  if (T > 0 && T <= kOneBlockTokens) {
+    const int waves = (int)((T + kWave - 1) / kWave);
+    route_one_kernel<<<dim3(1, (unsigned)L), dim3((unsigned)(waves < kChunks ? waves : kChunks) * kWave), 0, s>>>(
+        ids, ms, V, E, (int)T, expert_id, perm, inv_perm, counts, offsets);
+    return check_launch(name);
+  }
   if (nblk > 0) {
     route_count_kernel<<<dim3((unsigned)nblk, (unsigned)L), dim3(256), 0, s>>>(ids, ms, V, E, T, tpb, expert_id,
                                                                                 blk_counts);
