@@ -295,9 +295,20 @@ def pack_moe_weights(gate_w: torch.Tensor, up_w: torch.Tensor, down_w: torch.Ten
                      shared_down: Optional[torch.Tensor]) -> Tuple[torch.Tensor, torch.Tensor]:
     """Fresh (w_gu, w_down) operands holding copies of the given weights: gate_w/up_w
     [E, H, Ie] and down_w [E, Ie, H] are [in, out]; shared_* are nn.Linear weights
-    [out, in] (or None).  One strided copy per weight."""
+    [out, in] (or None).  One strided copy per weight, or one kernel for contiguous
+    weights without a shared block (cdx_moe_pack)."""
     E, H, ie = gate_w.shape
     has_shared = shared_gate is not None
+    ws = (gate_w, up_w, down_w)
+    if not has_shared and H % 64 == 0 and ie % 8 == 0 and 0 < E < 65536 and up_w.shape == gate_w.shape \
+            and down_w.shape == (E, ie, H) and all(w.is_cuda and w.dtype == torch.bfloat16 and w.is_contiguous()
+                                                   and w.device == gate_w.device and w.data_ptr() % 16 == 0 for w in ws):
+        P = padded_width(ie)
+        w_gu = torch.empty(E, 2, P, H, dtype=gate_w.dtype, device=gate_w.device)
+        w_down = torch.empty(E, H, P, dtype=gate_w.dtype, device=gate_w.device)
+        nat.check(nat.lib().cdx_moe_pack(*(w.data_ptr() for w in ws), E, H, ie, w_gu.data_ptr(), w_down.data_ptr(),
+                                         nat.stream_of(gate_w)), "cdx_moe_pack")
+        return w_gu, w_down
     w_gu, w_down = new_operands(E, H, ie, has_shared, gate_w.dtype, gate_w.device)
     views = operand_views(w_gu, w_down, ie, has_shared)
     with torch.no_grad():
@@ -395,8 +406,9 @@ def persistent_swiglu_cggr(sorted_tokens: torch.Tensor, gate_weights: torch.Tens
     identity permutation and no shared block; the gate/up products stay fp32 into
     the SwiGLU, which is rounded once (the reference rounds the two products to bf16
     first).  The operator holds no state, so the weights are copied into the kernel
-    layout on every call (three strided copies, about as many bytes as the GEMMs read;
-    a cache would miss writes made through ``.data``).  ``num_sms`` is accepted for
+    layout on every call (one kernel for contiguous weights, else three strided copies;
+    about as many bytes as the GEMMs read; a cache would miss writes made through
+    ``.data``).  ``num_sms`` is accepted for
     API compatibility."""
     forward_only("persistent_swiglu_cggr", sorted_tokens, gate_weights, up_weights, down_weights)
     nat.require_device(sorted_tokens, gate_weights, up_weights, down_weights, what="persistent_swiglu_cggr")

@@ -211,6 +211,15 @@ int cdx_moe_swiglu_residual_fwd(const uint16_t* x_dev, int64_t T, int32_t H, int
                                 uint16_t* residual_dev, void* stream);
 
 /*
+ * Copies expert weights gate, up [E][H][I] and down [E][I][H] ([in, out], the operator API's
+ * layout) into the operands above without a shared block: w_gu [E][2][P][H], w_down [E][H][P],
+ * units in [I, P) zeroed.  H % 64 == 0, I % 8 == 0, pointers 16-byte aligned.
+ * Replaces: cuda/persistent_cggr.py:479-530 (the weights of persistent_swiglu_cggr).
+ */
+int cdx_moe_pack(const uint16_t* gate_dev, const uint16_t* up_dev, const uint16_t* down_dev, int32_t E, int32_t H,
+                 int32_t I, uint16_t* w_gu_dev, uint16_t* w_down_dev, void* stream);
+
+/*
  * Grouped GEMM over expert segments of an already sorted token matrix:
  *   out[offsets[e]:offsets[e+1], :] = a[offsets[e]:offsets[e+1], :] @ W[e]
  * with W given K-contiguous: w_dev is [E][N][K] (W[e] transposed).  K % 64 == 0.
