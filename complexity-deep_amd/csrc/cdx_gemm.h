@@ -144,10 +144,13 @@ constexpr int kNumXcd = 8;
 // whose 256-row tiles leave most CUs idle.  The tile shape does not change any output
 // element's accumulation (the same MFMAs over the same K order), so every shape gives
 // the same bits.
+// WAVES_N of the four waves share the tile's columns: 2 (each wave half the rows and half
+// the columns), or 1 (a quarter of the rows, all columns) where an epilogue needs a wave to
+// hold whole heads of 128 columns of a 128-column tile.
 template <int BN_, int BK_, int STAGES_, int MINB_, int DMA_EVERY_ = 1, int DMA_OFF_ = 0, int READ_EVERY_ = 1,
-          int BM_ = kBM>
+          int BM_ = kBM, int WAVES_N_ = 2>
 struct GemmCfg {
-  static constexpr int BM = BM_, BN = BN_, BK = BK_, STAGES = STAGES_, MINB = MINB_;
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, STAGES = STAGES_, MINB = MINB_, WAVES_N = WAVES_N_;
   static constexpr int DMA_EVERY = DMA_EVERY_, DMA_OFF = DMA_OFF_, READ_EVERY = READ_EVERY_;
   static_assert(DMA_OFF < DMA_EVERY, "DMA slot offset must be below its spacing");
   static_assert(BM == 256 || BM == 128, "BM must be 128 or 256");
@@ -316,7 +319,7 @@ __global__ __launch_bounds__(kGemmThreads, Cfg::MINB) void gemm_nt_kernel(const 
   constexpr int RPL = 256 / ROW_BYTES;              // rows per 256-byte bank line (64 banks)
   constexpr int A_TILE_BYTES = kTM * ROW_BYTES;     // one stage of A
   constexpr int STAGE_BYTES = Cfg::STAGE_BYTES;     // A then B
-  constexpr int WM = kTM / 2, WN = kBN / 2;
+  constexpr int WM = kTM * Cfg::WAVES_N / 4, WN = kBN / Cfg::WAVES_N;
   constexpr int MI = WM / 16, NI = WN / 16;         // blocks of 16 x 16 per wave
   constexpr int ROWS_PER_DMA = 1024 / ROW_BYTES;    // rows one wave instruction fills
   constexpr int LD_A = kTM / ROWS_PER_DMA / 4;      // DMA instructions per wave and K step, A
@@ -339,7 +342,7 @@ __global__ __launch_bounds__(kGemmThreads, Cfg::MINB) void gemm_nt_kernel(const 
   const int lane = tid & 63;
   // Wave-uniform, so LDS addresses (the DMA's M0 in particular) stay scalar.
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / Cfg::WAVES_N, wn = wave % Cfg::WAVES_N;
 
   // ---- tile decode -------------------------------------------------------
   // Segment offsets are read clamped to [0, M] and a segment that ends before it

@@ -42,6 +42,12 @@ using XNarrowCfg = GemmCfg<64, 64, 3, 1, 2, 1, 1>;
 // slower (mu guidance 8.9 against 8.1 us).
 using SmallCfg = GemmCfg<128, 64, 3, 1, 2, 1, 1, 128>;
 using XSmallCfg = GemmCfg<64, 64, 3, 2, 1, 0, 1, 128>;
+// The 128-column tiles of mu-QKV + RoPE at head dim 128: every wave holds whole heads
+// (WAVES_N = 1).  With 256 x 256 tiles a 1B projection (4096 columns) of 400 tokens ran on
+// 32 of 256 CUs: 85.4 -> 35.8 us there, 84.4 -> 36.7 at 1024 tokens (128-row tiles),
+// 89.2 -> 62.4 at 2048 (256-row tiles).
+using NarrowHeadCfg = GemmCfg<128, 64, 3, 1, 4, 1, 1, kBM, 1>;
+using SmallHeadCfg = GemmCfg<128, 64, 3, 1, 2, 1, 1, 128, 1>;
 
 template <ALoad AL, Epi EP, class Cfg = DefaultCfg, int HD = 0>
 int launch(GemmParams p, hipStream_t s, const char* name) {
@@ -50,9 +56,11 @@ int launch(GemmParams p, hipStream_t s, const char* name) {
   if (nb == 0) return CDX_OK;
   // At most half as many 256 x 256 tiles as CUs (launch bound): half-width tiles give
   // twice the blocks, each with half the MFMA work per K step, still in one round.
-  // (A head of 128 columns does not fit a narrow tile's 64-column waves.)
-  if constexpr (Cfg::BN == 256 && (EP != Epi::kQKRope || HD <= 64)) {
-    if (2 * nb <= device_cu_count()) return launch<AL, EP, NarrowCfg, HD>(p, s, name);
+  // (A head of 128 columns does not fit a 64-column wave: NarrowHeadCfg.)
+  constexpr bool kHead128 = EP == Epi::kQKRope && HD == 128;
+  if constexpr (Cfg::BN == 256) {
+    using Narrow = std::conditional_t<kHead128, NarrowHeadCfg, NarrowCfg>;
+    if (2 * nb <= device_cu_count()) return launch<AL, EP, Narrow, HD>(p, s, name);
   }
   if constexpr (Cfg::BN == 128 && Cfg::BM == kBM && EP != Epi::kQKRope && EP != Epi::kSwiGLU) {
     if (2 * nb <= device_cu_count()) return launch<AL, EP, XNarrowCfg, HD>(p, s, name);
@@ -61,7 +69,7 @@ int launch(GemmParams p, hipStream_t s, const char* name) {
   // tile count is recounted for them (for the grouped passes, again an upper bound
   // with one partial tile per expert).
   if constexpr (Cfg::BM == kBM && Cfg::BN <= 128) {
-    using Small = std::conditional_t<Cfg::BN == 128, SmallCfg, XSmallCfg>;
+    using Small = std::conditional_t<Cfg::BN == 128, std::conditional_t<kHead128, SmallHeadCfg, SmallCfg>, XSmallCfg>;
     const bool grouped = p.offsets != nullptr && AL != ALoad::kSegmented;
     const int64_t mt_small = (p.M + Small::BM - 1) / Small::BM + (grouped ? p.E : 0);
     if (mt_small * p.nt_count <= (int64_t)Small::RESIDENT * device_cu_count()) {
