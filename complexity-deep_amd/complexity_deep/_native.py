@@ -10,12 +10,14 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib
 from pathlib import Path
 from typing import Callable, Optional
 
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libcdx.so"
+HOST_PATH = LIB_PATH.with_name("_host.so")
 
 _lib = None
 
@@ -142,6 +144,26 @@ def launch_region(name: str, device: torch.device, **shape):
     if hook is None:
         return _NO_REGION
     return _timed_region(hook, name, device, shape)
+
+
+_host = None
+
+
+def host():
+    """The operators' native call paths (module _host), or None while launches are timed (the
+    timing hook brackets the Python launch sites).  Each function takes the usual case of the
+    operator of its name and returns None for any other, having launched nothing."""
+    global _host
+    if _launch_hook is not None:
+        return None
+    if _host is None:
+        lib()
+        if not HOST_PATH.exists():
+            raise NativeLibraryMissing(
+                f"{HOST_PATH} is missing: build it with `python complexity-deep_amd/build_native.py` "
+                "(or __graft_entry__.build()); there is no fallback path")
+        _host = importlib.import_module("._host", __package__)
+    return _host
 
 
 def exported_symbols():

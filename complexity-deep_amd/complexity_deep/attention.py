@@ -386,12 +386,22 @@ class QKVWeights:
     def _linears(m):
         return (m.q_proj, m.k_proj, m.v_proj, m.mu_to_q, m.mu_to_k, m.mu_to_v)
 
-    def get(self, m) -> Tuple[torch.Tensor, torch.Tensor]:
-        ws = [lin.weight for lin in self._linears(m)]
+    _NAMES = ("q_proj", "k_proj", "v_proj", "mu_to_q", "mu_to_k", "mu_to_v")
+
+    def buffer(self, m) -> torch.Tensor:
+        """The [N, 2H] buffer, holding m's current weights."""
+        mods = m._modules
+        try:  # lin.weight of every projection, without nn.Module's attribute search
+            ws = [mods[n]._parameters["weight"] for n in self._NAMES]
+        except (KeyError, AttributeError):
+            ws = [lin.weight for lin in self._linears(m)]
         if self.buf is None or [w.data_ptr() for w in ws] != self.ptrs:
             self._bind(ws, m.hidden_size)
-        H = m.hidden_size
-        return self.buf[:, :H], self.buf[:, H:]
+        return self.buf
+
+    def get(self, m) -> Tuple[torch.Tensor, torch.Tensor]:
+        buf, H = self.buffer(m), m.hidden_size
+        return buf[:, :H], buf[:, H:]
 
     def _bind(self, ws, H: int) -> None:
         dt, dev = ws[0].dtype, ws[0].device
@@ -548,6 +558,17 @@ class ComplexityAttention(nn.Module):
         if attention_mask is None and not (self.training and self.attention_dropout > 0):
             cached = past_key_value is not None or use_cache
             fused = self.fused_prologue
+            fast = nat.host()
+            if fast is not None and (fused or self.other_head_dim) and hidden_states.is_cuda:
+                qn = (self.q_norm.weight, self.k_norm.weight) if self.use_qk_norm else (None, None)
+                pk, pv = past_key_value if past_key_value is not None else (None, None)
+                done = fast.attention(hidden_states, mu_prev, self._qkv_w.buffer(self), self.num_heads,
+                                      self.num_kv_heads, D, *qn, self.q_norm.eps if self.use_qk_norm else 0.0,
+                                      self.rotary_emb.cos_sin_table(past_len + S, hidden_states.device), pk, pv,
+                                      use_cache)
+                if done is not None:
+                    attn, k, v = done
+                    return self._out_proj(attn, residual), (k, v) if use_cache else None
             if fused and not cached and not few_rows(B * S, (self.num_heads + 2 * self.num_kv_heads) * D):
                 # Fused projection (V written transposed) and the causal GQA kernel, whose
                 # output is already merged over heads.

@@ -32,6 +32,11 @@ def mu_guidance(h: torch.Tensor, w: torch.Tensor, mu: torch.Tensor, mu_lo: float
     """clamp(h @ w^T + clamp(mu, mu_lo, mu_hi), lo, hi) through cdx_mu_guidance_fwd (fp32
     accumulate, one rounding).  h [..., H], w [H, H] and mu [H], all bf16.  ``out`` may be
     any [..., H] view with evenly spaced rows (e.g. the right half of a [T, 2H] buffer)."""
+    fast = nat.host()
+    if fast is not None:
+        done = fast.mu_guidance(h, w, mu, mu_lo, mu_hi, lo, hi, out)
+        if done is not None:
+            return done
     nat.require_device(h, w, mu, out, what="mu_guidance")
     H = h.shape[-1]
     h2 = h if h.is_contiguous() else h.contiguous()  # rows base + r * H

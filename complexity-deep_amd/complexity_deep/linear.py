@@ -23,6 +23,11 @@ from . import _native as nat
 
 def embedding(ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
     """table[ids] for int64 ids of any shape; returns [*ids.shape, H]."""
+    fast = nat.host()
+    if fast is not None:
+        out = fast.embedding(ids, table)
+        if out is not None:
+            return out
     nat.require_device(table, what="embedding")
     nat.require_device(ids, table, dtype=None, what="embedding")
     if table.dim() != 2:
@@ -45,6 +50,11 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     For N not a multiple of 8 the result is a view of the first N columns of a
     [rows, round_up(N, 8)] buffer (the kernel stores whole 16-byte pieces); its leading
     dimensions still merge (``.view(-1, N)`` works)."""
+    fast = nat.host()
+    if fast is not None:
+        out = fast.linear(x, w)
+        if out is not None:
+            return out
     nat.require_device(x, w, what="linear")
     N, K = w.shape
     if x.shape[-1] != K:
@@ -96,6 +106,9 @@ def linear_accumulate_(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor)
     """residual += x @ w^T in place with one rounding (a GEMM with beta = 1), for the shapes
     of few_rows.  x [..., K], w [N, K] and residual [..., N] contiguous; K % 64 == 0,
     N % 8 == 0."""
+    fast = nat.host()
+    if fast is not None and fast.linear_accumulate(x, w, residual):
+        return residual
     nat.require_device(x, w, residual, what="linear_accumulate_")
     N, K = w.shape
     if x.shape[-1] != K or residual.shape != x.shape[:-1] + (N,):

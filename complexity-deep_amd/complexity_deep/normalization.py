@@ -50,6 +50,11 @@ def add_rms_norm(x: torch.Tensor, residual: Optional[torch.Tensor], weight: torc
     residual=None gives a plain RMSNorm (second result None).  ``residual_out`` may
     be ``residual`` itself for an in-place update."""
     forward_only("add_rms_norm", x, residual, weight)
+    fast = nat.host()
+    if fast is not None and residual is not None and out is None and residual_out is None:
+        done = fast.add_rms_norm(x, residual, weight, eps, store_residual)
+        if done is not None:
+            return done
     nat.require_device(x, residual, what="add_rms_norm")
     shape = x.shape
     H = shape[-1]
@@ -84,9 +89,14 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6,
              out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Plain RMSNorm.  ``out`` may be any [..., H] view whose rows are evenly spaced, e.g.
     the left half of a [T, 2H] buffer (cdx_rmsnorm_ld_fwd writes rows at that stride)."""
+    forward_only("rms_norm", x, weight)
+    fast = nat.host()
+    if fast is not None:
+        y = fast.rms_norm(x, weight, eps, out)
+        if y is not None:
+            return y
     if out is None or out.is_contiguous():
         return add_rms_norm(x, None, weight, eps, out=out)[0]
-    forward_only("rms_norm", x, weight)
     nat.require_device(x, out, what="rms_norm")
     H = x.shape[-1]
     if out.shape != x.shape or out.dtype != x.dtype:

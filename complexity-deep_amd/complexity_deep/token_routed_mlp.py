@@ -58,6 +58,11 @@ def route_plan(ids: torch.Tensor, token_map: Optional[torch.Tensor], num_experts
 
     ids: int64 token ids (any shape) looked up through ``token_map`` (int64 [V]) after
     clamping to [0, V-1]; with token_map=None ``ids`` are expert ids already."""
+    fast = nat.host()
+    if fast is not None:
+        plan = fast.route_plan(ids, token_map, num_experts)
+        if plan is not None:
+            return RoutePlan(*plan, num_experts)
     nat.require_device(ids, token_map, dtype=None, what="route_plan")
     ids = ids.reshape(-1)
     if ids.dtype != torch.int64:
@@ -96,6 +101,11 @@ def route_plans(ids: torch.Tensor, token_maps: Sequence[torch.Tensor], num_exper
     L = len(token_maps)
     if L == 0:
         return []
+    fast = nat.host()
+    if fast is not None:
+        plans = fast.route_plans(ids, list(token_maps), num_experts)
+        if plans is not None:
+            return [RoutePlan(*p, num_experts) for p in plans]
     nat.require_device(ids, *token_maps, dtype=None, what="route_plans")
     V = token_maps[0].shape[0]
     maps = []
@@ -338,6 +348,11 @@ class MLPOperands:
         self.bufs: Optional[Tuple[torch.Tensor, torch.Tensor]] = None
         self.ptrs = None
 
+    def bound(self, ws) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+        """The operands if the weights ws (in the order last given to get) are still their
+        views, else None."""
+        return self.bufs if self.bufs is not None and [w.data_ptr() for w in ws] == self.ptrs else None
+
     def get(self, params: dict, E: int, H: int, ie: int, has_shared: bool) -> Tuple[torch.Tensor, torch.Tensor]:
         """params maps the operand_views names to the module's Parameters."""
         ws = list(params.values())
@@ -371,6 +386,11 @@ def moe_swiglu(x2d: torch.Tensor, plan: RoutePlan, w_gu: torch.Tensor, w_down: t
 def _moe_swiglu(x2d: torch.Tensor, perm: torch.Tensor, offsets: torch.Tensor, E: int, w_gu: torch.Tensor,
                 w_down: torch.Tensor, ie: int, has_shared: bool, residual: Optional[torch.Tensor] = None
                 ) -> torch.Tensor:
+    fast = nat.host()
+    if fast is not None:
+        done = fast.moe_swiglu(x2d, perm, offsets, E, w_gu, w_down, ie, has_shared, residual)
+        if done is not None:
+            return done
     T, H = x2d.shape
     P = padded_width(ie)
     nb = E + (1 if has_shared else 0)
@@ -488,6 +508,16 @@ class TokenRoutedMLP(nn.Module):
 
     def kernel_weights(self) -> Tuple[torch.Tensor, torch.Tensor]:
         """(w_gu, w_down): the operands the kernels read, of which the weights are views."""
+        p, mods = self._parameters, self._modules
+        try:  # the same weights as _weights(), without nn.Module's attribute search
+            ws = [p["gate_proj_w"], p["up_proj_w"], p["down_proj_w"]]
+            if self.use_shared_expert:
+                ws += [mods[n]._parameters["weight"] for n in ("shared_gate", "shared_up", "shared_down")]
+            bufs = self._operands.bound(ws)
+            if bufs is not None:
+                return bufs
+        except (KeyError, AttributeError):
+            pass  # a weight that is not a plain Parameter (parametrised, replaced)
         return self._operands.get(self._weights(), self.num_experts, self.hidden_size,
                                   self.expert_intermediate_size, self.use_shared_expert)
 

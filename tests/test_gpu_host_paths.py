@@ -1,0 +1,136 @@
+"""The operators' native call paths (complexity_deep._host) against the general Python paths
+they stand in for (taken while a timing hook is set): the same bits over the operand forms
+both accept (contiguous, strided, broadcast, cached), and the forms that the native paths
+leave to the general one (they return None and the call still works or raises)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+bf16 = torch.bfloat16
+
+
+def _both(fn):
+    from complexity_deep import _native as nat
+    with torch.no_grad():
+        a = fn()
+        nat.set_launch_hook(lambda *args: None)
+        try:
+            b = fn()
+        finally:
+            nat.set_launch_hook(None)
+    return a, b
+
+
+def _same(a, b, what):
+    if isinstance(a, torch.Tensor):
+        assert a.shape == b.shape and a.dtype == b.dtype and a.stride() == b.stride() and torch.equal(a, b), what
+    elif isinstance(a, (tuple, list)):
+        assert len(a) == len(b), what
+        for x, y in zip(a, b):
+            _same(x, y, what)
+    elif hasattr(a, "perm"):
+        _same([a.expert_id, a.perm, a.inv_perm, a.counts, a.offsets],
+              [b.expert_id, b.perm, b.inv_perm, b.counts, b.offsets], what)
+    else:
+        assert a == b, what
+
+
+def _new(*shape, seed=0):
+    g = torch.Generator().manual_seed(seed + sum(shape))
+    return torch.randn(*shape, generator=g).to(bf16).cuda()
+
+
+def test_operators(cdx):
+    from complexity_deep.layer import mu_guidance
+    from complexity_deep.linear import embedding, linear, linear_accumulate_
+    from complexity_deep.normalization import add_rms_norm, rms_norm
+    print("host paths: operators", flush=True)
+    x, r, w = _new(3, 7, 256), _new(3, 7, 256, seed=1), _new(256)
+    ids = torch.randint(-2, 503, (3, 7), device="cuda")
+    maps = [torch.randint(0, 5, (500,), device="cuda") for _ in range(2)]
+    wl, wm = _new(512, 256), _new(256, 256)
+
+    def pair(fn, half):
+        buf = torch.zeros(3, 7, 512, dtype=bf16, device="cuda")
+        fn(buf[..., :256] if half == 0 else buf[..., 256:])
+        return buf
+
+    cases = {
+        "rms_norm": lambda: rms_norm(x, w, 1e-6),
+        "rms_norm strided x": lambda: rms_norm(x.transpose(0, 1), w, 1e-6),
+        "rms_norm fp32 weight": lambda: rms_norm(x, w.float(), 1e-6),
+        "rms_norm out": lambda: pair(lambda o: rms_norm(x, w, 1e-6, out=o), 0),
+        "rms_norm empty": lambda: rms_norm(x[:0], w, 1e-6),
+        "add_rms_norm": lambda: add_rms_norm(x, r, w, 1e-6),
+        "add_rms_norm no residual kept": lambda: add_rms_norm(x, r, w, 1e-6, store_residual=False),
+        "add_rms_norm strided": lambda: add_rms_norm(x.transpose(0, 1), r.transpose(0, 1), w, 1e-6),
+        "embedding": lambda: embedding(ids.clamp(0, 255), wm),
+        "embedding int32": lambda: embedding(ids.clamp(0, 255).int(), wm),
+        "linear": lambda: linear(x, wl),
+        "linear ragged N": lambda: linear(x, wl[:509].contiguous()),
+        "linear strided x": lambda: linear(x.transpose(0, 1), wl),
+        "linear_accumulate_": lambda: linear_accumulate_(x, wm, r.clone()),
+        "mu_guidance": lambda: mu_guidance(x, wm, w, 0.0, 2.0, -2.0, 2.0),
+        "mu_guidance out": lambda: pair(lambda o: mu_guidance(x, wm, w, 0.0, 2.0, out=o), 1),
+        "mu_guidance strided": lambda: mu_guidance(x.transpose(0, 1), wm.t(), w),
+        "route_plan": lambda: cdx.route_plan(ids, maps[0], 5),
+        "route_plan int32 ids": lambda: cdx.route_plan(ids.int(), maps[0], 5),
+        "route_plan expert ids": lambda: cdx.route_plan(ids, None, 5),
+        "route_plan empty": lambda: cdx.route_plan(ids[:0], maps[0], 5),
+        "route_plans": lambda: cdx.route_plans(ids, maps, 5),
+        "route_plans int32 maps": lambda: cdx.route_plans(ids, [m.int() for m in maps], 5),
+    }
+    for what, fn in cases.items():
+        _same(*_both(fn), what)
+    for bad in (lambda: rms_norm(x, w[:8], 1e-6), lambda: linear(x, wl[:, :128].contiguous()),
+                lambda: mu_guidance(x, wm, w[:8]), lambda: add_rms_norm(x, r[:1], w, 1e-6),
+                lambda: rms_norm(x.cpu(), w, 1e-6), lambda: rms_norm(x.half(), w, 1e-6)):
+        with pytest.raises((RuntimeError, ValueError)):
+            bad()
+
+
+@pytest.mark.parametrize("H,nq,nkv", [(256, 4, 2), (320, 8, 4), (512, 4, 4)])
+def test_attention(cdx, H, nq, nkv):
+    print(f"host paths: attention H={H} heads={nq}/{nkv}", flush=True)
+    torch.manual_seed(H)
+    m = cdx.ComplexityAttention(H, nq, nkv).to(bf16).cuda().eval()
+    D = H // nq
+    pair = _new(2, 150, 2 * H)
+    row = _new(1, 1, H)
+    for S in (1, 5, 20, 150):
+        x, mu = pair[:, :S, :H], pair[:, :S, H:]  # evenly spaced rows for S = 150 only
+        kv = tuple(_new(2, nkv, 33, D, seed=s) for s in (3, 4))
+        for what, args in {"contiguous": (x.contiguous(), mu.contiguous()), "halves": (x, mu), "no mu": (x, None),
+                           "one mu row": (x.contiguous(), row.expand(2, S, H)), "mu of [1, S, H]": (x, mu[:1]),
+                           "mu per sequence": (x, mu[:, :1].expand(2, S, H))}.items():
+            for past in (None, kv):
+                for cache in (False, True):
+                    _same(*_both(lambda: m(args[0], mu_prev=args[1], past_key_value=past, use_cache=cache)),
+                          f"{what} S={S} past={past is not None} cache={cache}")
+
+
+def test_moe_and_model(cdx):
+    print("host paths: moe, model", flush=True)
+    torch.manual_seed(2)
+    moe = cdx.TokenRoutedMLP(256, 704, num_experts=4, vocab_size=500).to(bf16).cuda()
+    ids = torch.randint(0, 500, (3, 50), device="cuda")
+    x, r = _new(3, 50, 256), _new(3, 50, 256, seed=9)
+    for what, fn in {"moe": lambda: moe(x, token_ids=ids), "residual": lambda: moe(x, token_ids=ids, residual=r.clone()),
+                     "strided": lambda: moe(x.transpose(0, 1), token_ids=ids.t()), "average": lambda: moe(x)}.items():
+        _same(*_both(fn), what)
+    moe.up_proj_w.data.mul_(2)  # in place: seen by both
+    moe.gate_proj_w = torch.nn.Parameter(moe.gate_proj_w.detach().clone())  # replaced: bound again
+    _same(*_both(lambda: moe(x, token_ids=ids)), "after writes")
+    cfg = cdx.ComplexityConfig(vocab_size=500, hidden_size=256, intermediate_size=704, num_hidden_layers=3,
+                               num_attention_heads=4, num_key_value_heads=2, num_experts=4)
+    model = cdx.ComplexityModel(cfg).to(bf16).cuda().eval()
+    _same(*_both(lambda: model(ids).logits), "model")
+    _same(*_both(lambda: model(ids[:, :1]).logits), "model, one token")
+    with torch.no_grad():
+        past = model(ids, use_cache=True).past_key_values
+    a, b = _both(lambda: model(ids[:, -1:], past_key_values=past, use_cache=True))
+    _same(a.logits, b.logits, "step")
+    _same([t for kv in a.past_key_values for t in kv], [t for kv in b.past_key_values for t in kv], "step cache")
