@@ -42,6 +42,9 @@ using XNarrowCfg = GemmCfg<64, 64, 3, 1, 2, 1, 1>;
 // slower (mu guidance 8.9 against 8.1 us).
 using SmallCfg = GemmCfg<128, 64, 3, 1, 2, 1, 1, 128>;
 using XSmallCfg = GemmCfg<64, 64, 3, 2, 1, 0, 1, 128>;
+// 128 x 128 with two stages, two blocks per CU: a block's prologue and epilogue run beside the
+// other's K loop, and up to two tiles per CU finish together.
+using Small2Cfg = GemmCfg<128, 64, 2, 2, 2, 1, 1, 128>;
 // The 128-column tiles of mu-QKV + RoPE at head dim 128: every wave holds whole heads
 // (WAVES_N = 1).  With 256 x 256 tiles a 1B projection (4096 columns) of 400 tokens ran on
 // 32 of 256 CUs: 85.4 -> 35.8 us there, 84.4 -> 36.7 at 1024 tokens (128-row tiles),
@@ -49,8 +52,50 @@ using XSmallCfg = GemmCfg<64, 64, 3, 2, 1, 0, 1, 128>;
 using NarrowHeadCfg = GemmCfg<128, 64, 3, 1, 4, 1, 1, kBM, 1>;
 using SmallHeadCfg = GemmCfg<128, 64, 3, 1, 2, 1, 1, 128, 1>;
 
+// The tile for products of a size between one 128-row tile per CU and whole rounds of
+// 256 x 256 tiles.  0: the 256-row forms, 1: XSmallCfg, 2: SmallCfg, 3: Small2Cfg.  Grouped
+// passes count half a partial tile per expert.
+// Plain epilogues: the smallest tile that leaves at most one tile per CU (128 x 64 tiles at
+// two per CU lose to 128 x 128 ones at one: their LDS reads per MFMA are half as many again),
+// then two 128 x 128 tiles per CU.  One 256-row tile of M reads B once, so few rows stay with
+// the 256-row forms.  us, before -> here: mu guidance 2048 x 768 8.1 -> 8.1 (128 x 64), 3000 x
+// 1280 16.8 -> 15.4 (128 x 128), 4096 x 2048 35.4 -> 32.6 (two per CU); linear 1554 x 2560 x
+// 1920 27.3 -> 22.3; 200 x 768 x 32000 stays at 19.8 (two per CU: 22.4); MoE down passes 3001 x
+// 1792 x 1280 29.2 -> 21.6, 6000 rows 46.8 -> 30.6, 12000 rows stay at 51 (two per CU: 66).
+// SwiGLU: one 128 x 128 tile per CU where that is all (1000 tokens, 2048 wide: 42.0 -> 19.4),
+// else the cheaper of two tiles per CU, per tile 0.42 us a K step + 2.5, and rounds of
+// 256 x 256 tiles, 1.2 us a K step + 8 (fitted to 13 shapes within 15%): 2048 x 768 16.6 ->
+// 14.5, 8192 x 768 44.0 -> 36.9, 2048 x 2048 44.3 -> 30.9; 3001 x 1280 stays at 33.8 (36.1).
+template <ALoad AL, Epi EP, int HD>
+int mid_tile(const GemmParams& p) {
+  if (AL == ALoad::kSegmented || (EP == Epi::kQKRope && HD == 128)) return 0;
+  const int64_t cus = device_cu_count(), half_e = p.offsets != nullptr ? (p.E + 1) / 2 : 0;
+  const int64_t m128 = (p.M + 127) / 128 + half_e, n128 = (p.N + 127) / 128, t128 = m128 * n128;
+  // (The grouped count is an estimate: a twentieth over still fits one round as a rule.)
+  const int64_t once = p.offsets != nullptr ? cus + cus / 20 : cus;
+  if (EP == Epi::kSwiGLU) {
+    if (t128 <= once) return 2;
+    const int64_t t256 = ((p.M + 255) / 256 + half_e) * ((p.N + 255) / 256);
+    const double kt = p.K / 64, n = (double)t128 / cus;
+    const double two = n * (0.42 * kt + 2.5) + 5, square = (double)((t256 + cus - 1) / cus) * (1.2 * kt + 8);
+    return two < square ? 3 : 0;
+  }
+  if (EP != Epi::kQKRope && m128 * ((p.N + 63) / 64) <= cus) return 1;
+  if (t128 <= once) return 2;
+  return t128 <= 2 * cus && (p.M > kBM || p.offsets != nullptr) ? 3 : 0;
+}
+
 template <ALoad AL, Epi EP, class Cfg = DefaultCfg, int HD = 0>
 int launch(GemmParams p, hipStream_t s, const char* name) {
+  if constexpr (Cfg::BN == 256 && AL != ALoad::kSegmented && (EP != Epi::kQKRope || HD <= 64)) {
+    if (const int tile = mid_tile<AL, EP, HD>(p)) {
+      p.mt_count = (int32_t)((p.M + 127) / 128 + (p.offsets != nullptr ? p.E : 0));
+      if constexpr (EP != Epi::kQKRope && EP != Epi::kSwiGLU) {
+        if (tile == 1) return launch<AL, EP, XSmallCfg, HD>(p, s, name);
+      }
+      return tile == 2 ? launch<AL, EP, SmallCfg, HD>(p, s, name) : launch<AL, EP, Small2Cfg, HD>(p, s, name);
+    }
+  }
   p.nt_count = (p.N + Cfg::BN - 1) / Cfg::BN;
   const int64_t nb = (int64_t)p.mt_count * p.nt_count;
   if (nb == 0) return CDX_OK;
@@ -257,7 +302,9 @@ int moe_swiglu(const uint16_t* x, int64_t T, int32_t H, int32_t Ie, int32_t E, i
   const int64_t nt2 = cdiv(H, DefaultCfg::BN), cus = device_cu_count();
   const int64_t cost_expert = cdiv((cdiv(T, kBM) + E - 1) * nt2, cus) * (ks_shared + ks_expert);
   const int64_t cost_segmented = cdiv(cdiv(T, kBM) * nt2, cus) * (ks_shared + ks_expert) + ks_expert;
-  const bool segmented = cost_segmented < cost_expert;
+  // (Up to two 128 x 128 per-expert tiles per CU run as such, see mid_tile.)
+  const bool segmented = cost_segmented < cost_expert &&
+                         (cdiv(T, 128) + (E + 1) / 2) * cdiv(H, 128) > 2 * cus;
   // B: w_down [blocks][H][P]; the shared block (if any) serves K columns [0, P), the
   // token's expert block K columns [k_split, K).
   GemmParams p2{};
