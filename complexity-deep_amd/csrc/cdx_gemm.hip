@@ -61,27 +61,26 @@ using SmallHeadCfg = GemmCfg<128, 64, 3, 1, 2, 1, 1, 128, 1>;
 // the 256-row forms.  us, before -> here: mu guidance 2048 x 768 8.1 -> 8.1 (128 x 64), 3000 x
 // 1280 16.8 -> 15.4 (128 x 128), 4096 x 2048 35.4 -> 32.6 (two per CU); linear 1554 x 2560 x
 // 1920 27.3 -> 22.3; 200 x 768 x 32000 stays at 19.8 (two per CU: 22.4); MoE down passes 3001 x
-// 1792 x 1280 29.2 -> 21.6, 6000 rows 46.8 -> 30.6, 12000 rows stay at 51 (two per CU: 66).
-// SwiGLU: one 128 x 128 tile per CU where that is all (1000 tokens, 2048 wide: 42.0 -> 19.4),
+// 1792 x 1280 29.2 -> 27.6 (one tile per CU 21.6 while all fit one round, 33 with four over),
+// 6000 rows 46.8 -> 30.6, 12000 rows stay at 51 (two per CU: 66).
+// SwiGLU: one 128 x 128 tile per CU where that is all (400 tokens, 2048 wide: 30.9 -> 18.1),
 // else the cheaper of two tiles per CU, per tile 0.42 us a K step + 2.5, and rounds of
 // 256 x 256 tiles, 1.2 us a K step + 8 (fitted to 13 shapes within 15%): 2048 x 768 16.6 ->
-// 14.5, 8192 x 768 44.0 -> 36.9, 2048 x 2048 44.3 -> 30.9; 3001 x 1280 stays at 33.8 (36.1).
+// 14.5, 8192 x 768 44.0 -> 36.9, 1000 x 2048 42.0 -> 26.4, 2048 x 2048 44.3 -> 30.9; 3001 x 1280 stays at 33.8 (36.1).
 template <ALoad AL, Epi EP, int HD>
 int mid_tile(const GemmParams& p) {
   if (AL == ALoad::kSegmented || (EP == Epi::kQKRope && HD == 128)) return 0;
   const int64_t cus = device_cu_count(), half_e = p.offsets != nullptr ? (p.E + 1) / 2 : 0;
   const int64_t m128 = (p.M + 127) / 128 + half_e, n128 = (p.N + 127) / 128, t128 = m128 * n128;
-  // (The grouped count is an estimate: a twentieth over still fits one round as a rule.)
-  const int64_t once = p.offsets != nullptr ? cus + cus / 20 : cus;
   if (EP == Epi::kSwiGLU) {
-    if (t128 <= once) return 2;
+    if (t128 <= cus) return 2;
     const int64_t t256 = ((p.M + 255) / 256 + half_e) * ((p.N + 255) / 256);
     const double kt = p.K / 64, n = (double)t128 / cus;
     const double two = n * (0.42 * kt + 2.5) + 5, square = (double)((t256 + cus - 1) / cus) * (1.2 * kt + 8);
     return two < square ? 3 : 0;
   }
   if (EP != Epi::kQKRope && m128 * ((p.N + 63) / 64) <= cus) return 1;
-  if (t128 <= once) return 2;
+  if (t128 <= cus) return 2;
   return t128 <= 2 * cus && (p.M > kBM || p.offsets != nullptr) ? 3 : 0;
 }
 
