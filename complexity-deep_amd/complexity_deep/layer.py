@@ -126,7 +126,14 @@ class TransformerBlock(nn.Module):
                                           mu_prev=mu_prev)
         ln = self.post_attention_layernorm
         normed, h = add_rms_norm(attn_out, hidden_states, ln.weight, ln.eps)
-        h = h + self._mlp(normed, token_ids, None)
+        mlp = self.mlp
+        if type(mlp) in (TokenRoutedMLP, SwiGLU) and not (mlp._forward_hooks or mlp._forward_pre_hooks
+                                                          or nn.modules.module._has_any_global_hook()):
+            # h is this call's own tensor: the down pass adds its rows to it, with the
+            # roundings of the separate add (one 5 us pass less at 2048 tokens of 768).
+            h = self._mlp(normed, token_ids, None, residual=h)
+        else:
+            h = h + self._mlp(normed, token_ids, None)
         mu = self.mu_guidance(h) if self.mu_guidance is not None else None
         return h, new_kv, mu
 
