@@ -45,6 +45,8 @@ _SIGNATURES = {
                                           _vp, _vp]),
     "cdx_moe_swiglu_residual_fwd": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp,
                                                    _vp, _vp, _vp]),
+    "cdx_moe_swiglu_norm_residual_fwd": (ctypes.c_int, [_vp, _vp, ctypes.c_float, _i64, _i32, _i32, _i32, _i32, _vp,
+                                                        _vp, _vp, _vp, _vp, _vp]),
     "cdx_moe_pack": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp]),
     "cdx_grouped_gemm_fwd": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp]),
     "cdx_swiglu_fwd": (ctypes.c_int, [_vp, _vp, _i64, _i32, _i32, _vp, _vp]),
@@ -61,6 +63,9 @@ _SIGNATURES = {
     "cdx_qkv_cache_fwd": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _i32,
                                          _vp, _vp, ctypes.c_float, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp,
                                          ctypes.c_float, _vp, ctypes.c_size_t, _vp]),
+    "cdx_qkv_cache_norm_fwd": (ctypes.c_int, [_vp, _i64, _vp, ctypes.c_float, _vp, _i64, _vp, _vp, _i64, _i64, _i64,
+                                              _i32, _i32, _i32, _i32, _vp, _vp, ctypes.c_float, _vp, _i64, _vp, _vp,
+                                              _i64, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, ctypes.c_size_t, _vp]),
     "cdx_vt_pack": (ctypes.c_int, [_vp, _i64, _i64, _i64, _i32, _vp, _i64, _vp]),
     "cdx_attention_cache_fwd": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _i64,
                                                ctypes.c_float, _vp, _vp]),

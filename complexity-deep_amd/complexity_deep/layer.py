@@ -20,7 +20,7 @@ import torch.nn.functional as F
 
 from . import _native as nat
 from ._grad import forward_only
-from .attention import ComplexityAttention
+from .attention import ComplexityAttention, _plain_linear
 from .mlp import SwiGLU
 from .normalization import RMSNorm, add_rms_norm, rms_norm
 from .token_routed_mlp import RoutePlan, TokenRoutedMLP
@@ -169,3 +169,41 @@ class TransformerBlock(nn.Module):
             normed = rms_norm(h, next_norm.weight, next_norm.eps)
         mu = self.mu_guidance.fused(h, -2.0, 2.0, out=mu_out) if (want_mu and self.mu_guidance is not None) else None
         return h, normed, new_kv, mu
+
+    def step(self, h: torch.Tensor, mu_prev: Optional[torch.Tensor], past, route: Optional[RoutePlan],
+             want_mu: bool = True):
+        """One block of a generation step of at most 8 rows, h updated in place: what
+        forward_fused computes without a mask, with both norms folded into the products
+        that read them.  Returns (new_kv, mu), or None, nothing having run, if the block is
+        not the plain one (a replaced or hooked submodule, a dense MLP) or the operands are
+        not the usual ones."""
+        fast = nat.host()
+        attn, mlp = self.self_attn, self.mlp
+        ln1, ln2 = self.input_layernorm, self.post_attention_layernorm
+        if (fast is None or route is None or type(self).forward_fused is not _FORWARD_FUSED
+                or type(attn) is not ComplexityAttention or type(mlp) is not TokenRoutedMLP
+                or type(ln1) is not RMSNorm or type(ln2) is not RMSNorm or not _plain_linear(attn.o_proj)
+                or attn._forward_hooks or attn._forward_pre_hooks or mlp._forward_hooks or mlp._forward_pre_hooks
+                or (attn.training and attn.attention_dropout > 0) or not (attn.fused_prologue or attn.other_head_dim)):
+            return None
+        guide = self.mu_guidance if want_mu else None
+        if guide is not None and type(guide) is not MuGuidance:
+            return None
+        qn, kn = (attn.q_norm, attn.k_norm) if attn.use_qk_norm else (None, None)
+        pk, pv = past if past is not None else (None, None)
+        n_pos = h.shape[1] + (pk.shape[2] if pk is not None else 0)
+        w_gu, w_down = mlp.kernel_weights()
+        done = fast.block_step(
+            h, ln1.weight, ln1.eps, mu_prev, attn._qkv_w.buffer(attn), attn.num_heads, attn.num_kv_heads, attn.head_dim,
+            qn.weight if qn is not None else None, kn.weight if kn is not None else None, qn.eps if qn is not None else 0.0,
+            attn.rotary_emb.cos_sin_table(n_pos, h.device), pk, pv, attn.o_proj.weight, ln2.weight, ln2.eps, route.perm,
+            route.offsets, route.num_experts, w_gu, w_down, mlp.expert_intermediate_size, mlp.use_shared_expert,
+            guide.mu_proj.weight if guide is not None else None, guide.mu if guide is not None else None,
+            guide.mu_min if guide is not None else 0.0, guide.mu_max if guide is not None else 0.0, -2.0, 2.0)
+        if done is None:
+            return None
+        k, v, mu = done
+        return (k, v), mu
+
+
+_FORWARD_FUSED = TransformerBlock.forward_fused

@@ -221,25 +221,38 @@ class ComplexityModel(nn.Module):
         mu_prev = self.mu_init.expand(B, S, -1) if self.config.use_mu_guidance else None
         plans = self.route_plans(input_ids)
         new_kvs = [] if use_cache else None
-        n_layers = len(self.layers)
-        normed = rms_norm(h, self.layers[0].input_layernorm.weight, self.layers[0].input_layernorm.eps) \
-            if n_layers else rms_norm(h, self.norm.weight, self.norm.eps)
+        layers = list(self.layers)
+        n_layers = len(layers)
+        # A generation step of a few rows runs block by block through TransformerBlock.step,
+        # which takes h itself (its norms are folded); other calls hand each block its
+        # normalised input, produced by the block before.
+        steps = attention_mask is None and 0 < B * S <= 8
+        normed = None
         # Layers 1.. read their normalised input and mu side by side from one [B, S, 2H]
         # buffer, written by the layer before (one K = 2H operand for the projection).
         pair = torch.empty(B, S, 2 * h.shape[-1], dtype=h.dtype, device=h.device) \
-            if self.config.use_mu_guidance and n_layers > 1 else None
-        for i, layer in enumerate(self.layers):
+            if self.config.use_mu_guidance and n_layers > 1 and not steps else None
+        for i, layer in enumerate(layers):
             last = i + 1 == n_layers
-            next_norm = self.norm if last else self.layers[i + 1].input_layernorm
-            h, normed, new_kv, mu = layer.forward_fused(
-                h, normed, next_norm, attention_mask=attention_mask,
-                past_key_value=past_key_values[i] if past_key_values is not None else None,
-                use_cache=use_cache, token_ids=input_ids, mu_prev=mu_prev, route=plans[i],
-                want_mu=not last, pair=None if last else pair)
+            past = past_key_values[i] if past_key_values is not None else None
+            done = layer.step(h, mu_prev, past, plans[i], want_mu=not last) if steps else None
+            if done is not None:
+                new_kv, mu = done
+                normed = None
+            else:
+                if normed is None:
+                    normed = rms_norm(h, layer.input_layernorm.weight, layer.input_layernorm.eps)
+                next_norm = self.norm if last else layers[i + 1].input_layernorm
+                h, normed, new_kv, mu = layer.forward_fused(
+                    h, normed, next_norm, attention_mask=attention_mask, past_key_value=past,
+                    use_cache=use_cache, token_ids=input_ids, mu_prev=mu_prev, route=plans[i],
+                    want_mu=not last, pair=None if last else pair)
             if mu is not None:
                 mu_prev = mu  # clamped to [-2, 2] inside the mu-guidance kernel
             if use_cache:
                 new_kvs.append(new_kv)
+        if normed is None:
+            normed = rms_norm(h, self.norm.weight, self.norm.eps)
         logits = linear(normed, self.lm_head.weight)
         loss = None
         if labels is not None:

@@ -240,7 +240,8 @@ namespace {
 // Both MoE passes; with `residual`, the down pass adds its rows to `out` in place.
 int moe_swiglu(const uint16_t* x, int64_t T, int32_t H, int32_t Ie, int32_t E, int32_t has_shared,
                const int32_t* perm, const int32_t* offsets, const uint16_t* w_gu, const uint16_t* w_down,
-               uint16_t* inter, uint16_t* out, void* stream, bool residual, const char* name) {
+               uint16_t* inter, uint16_t* out, void* stream, bool residual, const char* name,
+               const uint16_t* norm_w = nullptr, float eps = 0.f) {
   clear_error();
   if (T < 0 || T > INT32_MAX || H <= 0 || Ie <= 0 || E <= 0 || E > 64)
     return fail(CDX_EINVAL, "%s: bad shape T=%lld H=%d Ie=%d E=%d", name, (long long)T, H, Ie, E);
@@ -262,8 +263,9 @@ int moe_swiglu(const uint16_t* x, int64_t T, int32_t H, int32_t Ie, int32_t E, i
     return fail(CDX_EUNSUPPORTED, "%s: the gate/up weights must fit 4 GB (E=%d, P=%d, H=%d)", name, E, P, H);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (T <= kSkinnyRows)
-    return skinny_moe(x, (int32_t)T, H, P, E, has_shared != 0, perm, offsets, w_gu, w_down, inter, out, residual, s,
-                      name);
+    return skinny_moe(x, (int32_t)T, H, P, E, has_shared != 0, perm, offsets, w_gu, w_down, inter, out, residual,
+                      norm_w, eps, s, name);
+  if (norm_w != nullptr) return fail(CDX_EUNSUPPORTED, "%s: a folded norm needs T <= 8", name);
   const int32_t mt = (int32_t)(cdiv(T, kBM) + E);
 
   // Pass 1: gathered rows x[perm] times the gate/up rows of the shared block and the
@@ -349,6 +351,19 @@ extern "C" int cdx_moe_swiglu_residual_fwd(const uint16_t* x, int64_t T, int32_t
                                            uint16_t* residual, void* stream) {
   return cdx::moe_swiglu(x, T, H, Ie, E, has_shared, perm, offsets, w_gu, w_down, inter, residual, stream, true,
                          "cdx_moe_swiglu_residual_fwd");
+}
+
+extern "C" int cdx_moe_swiglu_norm_residual_fwd(uint16_t* h, const uint16_t* norm_w, float eps, int64_t T, int32_t H,
+                                                int32_t Ie, int32_t E, int32_t has_shared, const int32_t* perm,
+                                                const int32_t* offsets, const uint16_t* w_gu, const uint16_t* w_down,
+                                                uint16_t* inter, void* stream) {
+  using namespace cdx;
+  const char* name = "cdx_moe_swiglu_norm_residual_fwd";
+  clear_error();
+  if (!(eps >= 0.f)) return fail(CDX_EINVAL, "%s: eps must be >= 0", name);
+  if (T > kNormRows) return fail(CDX_EUNSUPPORTED, "%s: T=%lld must be <= %d", name, (long long)T, kNormRows);
+  if (T > 0 && (!norm_w || !aligned16(norm_w))) return fail(CDX_EINVAL, "%s: bad norm weight pointer", name);
+  return moe_swiglu(h, T, H, Ie, E, has_shared, perm, offsets, w_gu, w_down, inter, h, stream, true, name, norm_w, eps);
 }
 
 extern "C" int cdx_grouped_gemm_fwd(const uint16_t* a, int64_t T, int32_t K, int32_t N, int32_t E,

@@ -242,16 +242,16 @@ extern "C" size_t cdx_qkv_cache_workspace_bytes(int64_t B, int64_t S, int32_t nq
   return (size_t)(M * N) * (cdx::skinny_fits(M, N) ? sizeof(float) : sizeof(uint16_t));
 }
 
-extern "C" int cdx_qkv_cache_fwd(const uint16_t* x, int64_t ldx, const uint16_t* mu, int64_t ldmu, const uint16_t* w,
-                                 const uint16_t* w_mu, int64_t ldw, int64_t B, int64_t S, int32_t H, int32_t nq,
-                                 int32_t nkv, int32_t hd, const uint16_t* q_norm_w, const uint16_t* k_norm_w,
-                                 float eps, const float* cos_sin, int64_t n_pos, const uint16_t* past_k,
-                                 const uint16_t* past_v, int64_t past, uint16_t* q_out, uint16_t* k_out,
-                                 uint16_t* v_out, uint16_t* attn_out, float scale, void* work, size_t work_bytes,
-                                 void* stream) {
-  using namespace cdx;
+namespace cdx {
+namespace {
+
+int qkv_cache(const char* name, const uint16_t* x_norm_w, float x_eps, const uint16_t* x, int64_t ldx,
+              const uint16_t* mu, int64_t ldmu, const uint16_t* w, const uint16_t* w_mu, int64_t ldw, int64_t B,
+              int64_t S, int32_t H, int32_t nq, int32_t nkv, int32_t hd, const uint16_t* q_norm_w,
+              const uint16_t* k_norm_w, float eps, const float* cos_sin, int64_t n_pos, const uint16_t* past_k,
+              const uint16_t* past_v, int64_t past, uint16_t* q_out, uint16_t* k_out, uint16_t* v_out,
+              uint16_t* attn_out, float scale, void* work, size_t work_bytes, void* stream) {
   clear_error();
-  const char* name = "cdx_qkv_cache_fwd";
   if (B < 0 || S < 0 || H <= 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || past < 0 || n_pos < 0)
     return fail(CDX_EINVAL, "%s: bad shape B=%lld S=%lld H=%d nq=%d nkv=%d past=%lld", name, (long long)B,
                 (long long)S, H, nq, nkv, (long long)past);
@@ -291,6 +291,8 @@ extern "C" int cdx_qkv_cache_fwd(const uint16_t* x, int64_t ldx, const uint16_t*
 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool few = skinny_fits(M, N);
+  if (x_norm_w && (!few || M > kNormRows))
+    return fail(CDX_EUNSUPPORTED, "%s: a folded norm needs B * S <= %d", name, kNormRows);
   if (few) {
     SkinnyParams sp{};
     sp.a = x;
@@ -306,6 +308,8 @@ extern "C" int cdx_qkv_cache_fwd(const uint16_t* x, int64_t ldx, const uint16_t*
     sp.K = mu ? 2 * H : H;
     sp.c = work;
     sp.ldc = N;
+    sp.norm_w = x_norm_w;
+    sp.eps = x_eps;
     if (int rc = skinny_gemm(sp, SkinnyEpi::kF32, s, name)) return rc;
   } else if (int rc = cdx_mu_qkv_fwd(x, ldx, mu, ldmu, w, w_mu, ldw, M, H, (int32_t)N, static_cast<uint16_t*>(work), N,
                                      stream)) {
@@ -338,6 +342,39 @@ extern "C" int cdx_qkv_cache_fwd(const uint16_t* x, int64_t ldx, const uint16_t*
   else
     qkv_cache_kernel<uint16_t><<<grid, dim3(256), 0, s>>>(p);
   return check_launch(name);
+}
+
+}  // namespace
+}  // namespace cdx
+
+extern "C" int cdx_qkv_cache_fwd(const uint16_t* x, int64_t ldx, const uint16_t* mu, int64_t ldmu, const uint16_t* w,
+                                 const uint16_t* w_mu, int64_t ldw, int64_t B, int64_t S, int32_t H, int32_t nq,
+                                 int32_t nkv, int32_t hd, const uint16_t* q_norm_w, const uint16_t* k_norm_w,
+                                 float eps, const float* cos_sin, int64_t n_pos, const uint16_t* past_k,
+                                 const uint16_t* past_v, int64_t past, uint16_t* q_out, uint16_t* k_out,
+                                 uint16_t* v_out, uint16_t* attn_out, float scale, void* work, size_t work_bytes,
+                                 void* stream) {
+  return cdx::qkv_cache("cdx_qkv_cache_fwd", nullptr, 0.f, x, ldx, mu, ldmu, w, w_mu, ldw, B, S, H, nq, nkv, hd,
+                        q_norm_w, k_norm_w, eps, cos_sin, n_pos, past_k, past_v, past, q_out, k_out, v_out, attn_out,
+                        scale, work, work_bytes, stream);
+}
+
+extern "C" int cdx_qkv_cache_norm_fwd(const uint16_t* h, int64_t ldh, const uint16_t* norm_w, float norm_eps,
+                                      const uint16_t* mu, int64_t ldmu, const uint16_t* w, const uint16_t* w_mu,
+                                      int64_t ldw, int64_t B, int64_t S, int32_t H, int32_t nq, int32_t nkv,
+                                      int32_t hd, const uint16_t* q_norm_w, const uint16_t* k_norm_w, float eps,
+                                      const float* cos_sin, int64_t n_pos, const uint16_t* past_k,
+                                      const uint16_t* past_v, int64_t past, uint16_t* q_out, uint16_t* k_out,
+                                      uint16_t* v_out, uint16_t* attn_out, float scale, void* work,
+                                      size_t work_bytes, void* stream) {
+  using namespace cdx;
+  const char* name = "cdx_qkv_cache_norm_fwd";
+  clear_error();
+  if (!norm_w || !aligned16(norm_w)) return fail(CDX_EINVAL, "%s: bad norm weight pointer", name);
+  if (!(norm_eps >= 0.f)) return fail(CDX_EINVAL, "%s: eps must be >= 0", name);
+  return qkv_cache(name, norm_w, norm_eps, h, ldh, mu, ldmu, w, w_mu, ldw, B, S, H, nq, nkv, hd, q_norm_w, k_norm_w,
+                   eps, cos_sin, n_pos, past_k, past_v, past, q_out, k_out, v_out, attn_out, scale, work, work_bytes,
+                   stream);
 }
 
 extern "C" int cdx_vt_pack(const uint16_t* v, int64_t slabs, int64_t rows, int64_t S, int32_t hd, uint16_t* vt,

@@ -9,6 +9,9 @@ namespace cdx {
 // Rows up to which the skinny kernels may replace the tile engine (cdx_gemm.h).
 constexpr int kSkinnyRows = 64;
 
+// Rows up to which a product can take its A operand through an RMSNorm.
+constexpr int kNormRows = 8;
+
 // Whether a product of M rows and N columns runs faster here.  Past 16 rows every block of
 // columns re-reads A from L2, which costs in proportion to row groups x column blocks: the
 // line lies at 4 per CU (measured on 256 CUs, K = 2048, here against the tile engine: 32
@@ -34,14 +37,20 @@ struct SkinnyParams {
   int64_t ldc;
   const uint16_t* bias;  // kBiasClamp: c = clamp(acc + clamp(bias[n], bias_lo, bias_hi), lo, hi)
   float bias_lo, bias_hi, lo, hi;
+  // Not null (kF32, M <= kNormRows): columns [0, k_split) of A are RMSNorm(a) with these
+  // weights and eps.
+  const uint16_t* norm_w;
+  float eps;
 };
 
 // For shapes that fit (skinny_fits); operands 16-byte aligned, leading dimensions multiples of 8.
 int skinny_gemm(const SkinnyParams& p, SkinnyEpi epi, hipStream_t s, const char* name);
 
-// Both MoE passes for 1 <= T <= kSkinnyRows tokens (arguments as cdx_moe_swiglu_fwd).
+// Both MoE passes for 1 <= T <= kSkinnyRows tokens (arguments as cdx_moe_swiglu_fwd); with
+// norm_w (T <= kNormRows) of RMSNorm(x).  x may be `out` itself with norm_w and residual: the
+// gate/up pass is done with it before the down pass adds to it.
 int skinny_moe(const uint16_t* x, int32_t T, int32_t H, int32_t P, int32_t E, bool shared, const int32_t* perm,
                const int32_t* offsets, const uint16_t* w_gu, const uint16_t* w_down, uint16_t* inter, uint16_t* out,
-               bool residual, hipStream_t s, const char* name);
+               bool residual, const uint16_t* norm_w, float eps, hipStream_t s, const char* name);
 
 }  // namespace cdx

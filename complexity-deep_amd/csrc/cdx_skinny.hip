@@ -69,12 +69,46 @@ struct Item {
   }
 };
 
+// RMSNorm folded into the A operand (M <= 8): the operand becomes bf16(weight * x) and the
+// row's 1 / rms, a factor of the whole sum, is applied to the fp32 result, so the norm costs
+// no pass of its own.  Every block reads all of x anyway and sums its squares on the way.
+// (A separate norm rounds weight * x / rms to bf16 instead: the same relative rounding.)
+__device__ __forceinline__ bf16x8 norm_frag(bf16x8 x, const uint4& w, float& ss) {
+  float a[8], b[8];
+  unpack8(__builtin_bit_cast(uint4, x), a);
+  unpack8(w, b);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    ss = __builtin_fmaf(a[i], a[i], ss);
+    a[i] *= b[i];
+  }
+  return __builtin_bit_cast(bf16x8, pack8(a));
+}
+// Each lane's sum of squares to the sum of its row (HALF: lanes l, l ^ 8, l ^ 16, l ^ 32 ...
+// hold the row's columns), kept per wave in LDS.
+__device__ __forceinline__ void row_squares(float ss, float* out, int lane) {
+#pragma unroll
+  for (int d = 8; d < 64; d <<= 1) ss += __shfl_xor(ss, d, 64);
+  if (lane < 8) out[lane] = ss;
+}
+template <int W>
+__device__ __forceinline__ float row_scale(const float* squares, int m, int K, float eps) {
+  float t = 0.f;
+#pragma unroll
+  for (int w = 0; w < W; ++w) t += squares[w * 8 + m];
+  return rsqrtf(t / (float)K + eps);
+}
+
 // CH: 64-column chunks of K loaded before their MFMAs run (the loads in flight per wave).
-template <int MT, int NB, int W, int CH, bool HALF, SkinnyEpi EPI>
+// NORM: columns [0, k_split) of A enter as RMSNorm(a) (see norm_frag); their sums are kept
+// apart from the second source's until the scale is applied.
+template <int MT, int NB, int W, int CH, bool HALF, SkinnyEpi EPI, bool NORM = false>
 __global__ __launch_bounds__(64 * W) void skinny_kernel(const SkinnyParams p) {
   using Sh = Shape<HALF>;
   constexpr int NS = Sh::kSub;
-  __shared__ f32x4 red[W * NB * MT * 64];
+  static_assert(!NORM || (HALF && MT == 1), "the folded norm is for M <= 8");
+  __shared__ f32x4 red[W * NB * MT * 64 * (NORM ? 2 : 1)];
+  __shared__ float squares[NORM ? W * 8 : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = Sh::row(lane), ko = Sh::k_off(lane);
@@ -96,6 +130,10 @@ __global__ __launch_bounds__(64 * W) void skinny_kernel(const SkinnyParams p) {
   for (int i = 0; i < NB; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 acc_n[NORM ? NB : 1];  // NORM: the sums of the normalised columns, unscaled
+#pragma unroll
+  for (int i = 0; i < (NORM ? NB : 1); ++i) acc_n[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float ss = 0.f;
 
   // This wave's chunks of 64 columns: one contiguous run.
   const int chunks = p.K >> 6;
@@ -103,11 +141,15 @@ __global__ __launch_bounds__(64 * W) void skinny_kernel(const SkinnyParams p) {
   const int c_end = min(chunks, (wave + 1) * per);
   for (int c0 = wave * per; c0 < c_end; c0 += CH) {
     bf16x8 bf[CH][NS][NB], af[CH][NS][MT];
+    uint4 nw[NORM ? CH : 1];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       if (c0 + u >= c_end) break;
       const int k = (c0 + u) << 6;
       const bool second = k >= p.k_split;
+      if constexpr (NORM) {
+        if (!second) nw[u] = *reinterpret_cast<const uint4*>(p.norm_w + k + ko);
+      }
       const uint16_t* bk = (second ? p.b2 : p.b) + (second ? k - p.k_split : k);
       const uint16_t* ak = (second ? p.a2 : p.a) + (second ? k - p.k_split : k);
 #pragma unroll
@@ -122,6 +164,14 @@ __global__ __launch_bounds__(64 * W) void skinny_kernel(const SkinnyParams p) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       if (c0 + u >= c_end) break;
+      if constexpr (NORM) {
+        if (((c0 + u) << 6) < p.k_split) {
+          const bf16x8 x = norm_frag(af[u][0][0], nw[u], ss);
+#pragma unroll
+          for (int i = 0; i < NB; ++i) acc_n[i] = mfma16(bf[u][0][i], x, acc_n[i]);
+          continue;
+        }
+      }
 #pragma unroll
       for (int s = 0; s < NS; ++s)
 #pragma unroll
@@ -135,6 +185,11 @@ __global__ __launch_bounds__(64 * W) void skinny_kernel(const SkinnyParams p) {
   for (int i = 0; i < NB; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j) red[(wave * NB * MT + i * MT + j) * 64 + lane] = acc[i][j];
+  if constexpr (NORM) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) red[((W + wave) * NB + i) * 64 + lane] = acc_n[i];
+    row_squares(ss, squares + wave * 8, lane);
+  }
   __syncthreads();
   using It = Item<HALF>;
   for (int i = threadIdx.x; i < NB * MT * It::kItems; i += 64 * W) {
@@ -143,7 +198,9 @@ __global__ __launch_bounds__(64 * W) void skinny_kernel(const SkinnyParams p) {
     const int m = (blk % MT) * 16 + it.m;
     const int n = n0 + (blk / MT) * Sh::kRows + 4 * it.q;
     if (m >= p.M || n >= ((p.N + 7) & ~7)) continue;
-    const f32x4 t = it.template total<NB * MT, W>(red, blk);
+    f32x4 t = it.template total<NB * MT, W>(red, blk);
+    if constexpr (NORM)
+      t += it.template total<NB, W>(red + W * NB * 64, blk) * row_scale<W>(squares, m, p.k_split, p.eps);
     float y[4] = {t[0], t[1], t[2], t[3]};
     if constexpr (EPI == SkinnyEpi::kF32) {
       *reinterpret_cast<float4*>(static_cast<float*>(p.c) + (int64_t)m * p.ldc + n) = make_float4(y[0], y[1], y[2], y[3]);
@@ -176,6 +233,12 @@ template <int MT, int NB, int W, int CH, bool HALF>
 int launch_skinny(const SkinnyParams& p, SkinnyEpi epi, hipStream_t s, const char* name) {
   constexpr int kCols = Shape<HALF>::kRows * NB;
   const dim3 grid((unsigned)((p.N + kCols - 1) / kCols)), block(64 * W);
+  if constexpr (HALF) {
+    if (p.norm_w != nullptr) {  // (skinny_gemm: kF32 only)
+      skinny_kernel<MT, NB, W, CH, HALF, SkinnyEpi::kF32, true><<<grid, block, 0, s>>>(p);
+      return check_launch(name);
+    }
+  }
   switch (epi) {
     case SkinnyEpi::kStore: skinny_kernel<MT, NB, W, CH, HALF, SkinnyEpi::kStore><<<grid, block, 0, s>>>(p); break;
     case SkinnyEpi::kBiasClamp:
@@ -205,16 +268,21 @@ struct SkinnyMoeParams {
   uint16_t* out;           // [T][H], rows in token order
   int32_t T, H, P, E;
   int32_t shared;          // 1: block 0 is the shared expert
+  const uint16_t* norm_w;  // not null (T <= 8): the gate/up pass reads RMSNorm(x)
+  float eps;
 };
 
 // Gate/up: block (unit group, weight block).  The gate and up rows of 16 (HALF: 8) units of
 // one weight block times the rows of its segment, SwiGLU in the epilogue.  A routed expert
 // without tokens reads nothing.
-template <int MT, int W, int CH, bool HALF>
+template <int MT, int W, int CH, bool HALF, bool NORM = false>
 __global__ __launch_bounds__(64 * W) void skinny_gate_up_kernel(const SkinnyMoeParams p) {
   using Sh = Shape<HALF>;
   constexpr int NS = Sh::kSub;
+  static_assert(!NORM || (HALF && MT == 1), "the folded norm is for T <= 8");
   __shared__ f32x4 red[W * 2 * MT * 64];
+  __shared__ float squares[NORM ? W * 8 : 1];
+  float ss = 0.f;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = Sh::row(lane), ko = Sh::k_off(lane);
@@ -245,10 +313,12 @@ __global__ __launch_bounds__(64 * W) void skinny_gate_up_kernel(const SkinnyMoeP
   const int c_end = min(chunks, (wave + 1) * per);
   for (int c0 = wave * per; c0 < c_end; c0 += CH) {
     bf16x8 wf[CH][NS][2], xf[CH][NS][MT];
+    uint4 nw[NORM ? CH : 1];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       if (c0 + u >= c_end) break;
       const int k = (c0 + u) << 6;
+      if constexpr (NORM) nw[u] = *reinterpret_cast<const uint4*>(p.norm_w + k + ko);
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         wf[u][s][0] = ld8(gate + k + 32 * s);
@@ -272,6 +342,7 @@ __global__ __launch_bounds__(64 * W) void skinny_gate_up_kernel(const SkinnyMoeP
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       if (c0 + u >= c_end) break;
+      if constexpr (NORM) xf[u][0][0] = norm_frag(xf[u][0][0], nw[u], ss);
 #pragma unroll
       for (int s = 0; s < NS; ++s)
 #pragma unroll
@@ -286,6 +357,7 @@ __global__ __launch_bounds__(64 * W) void skinny_gate_up_kernel(const SkinnyMoeP
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j) red[(wave * 2 * MT + i * MT + j) * 64 + lane] = acc[i][j];
+  if constexpr (NORM) row_squares(ss, squares + wave * 8, lane);
   __syncthreads();
   const int S = 1 + p.shared;
   const int col0 = (is_shared ? 0 : p.shared * p.P) + u0;
@@ -295,8 +367,13 @@ __global__ __launch_bounds__(64 * W) void skinny_gate_up_kernel(const SkinnyMoeP
     const It it(i % It::kItems);
     const int pos = s0 + j * 16 + it.m;
     if (pos >= s1) continue;
-    const f32x4 gv = it.template total<2 * MT, W>(red, j);
-    const f32x4 uv = it.template total<2 * MT, W>(red, MT + j);
+    f32x4 gv = it.template total<2 * MT, W>(red, j);
+    f32x4 uv = it.template total<2 * MT, W>(red, MT + j);
+    if constexpr (NORM) {
+      const float rs = row_scale<W>(squares, it.m, p.H, p.eps);
+      gv *= rs;
+      uv *= rs;
+    }
     float y[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) y[v] = silu_f32(gv[v]) * uv[v];
@@ -427,8 +504,11 @@ __global__ __launch_bounds__(64 * W) void skinny_down_kernel(const SkinnyMoePara
 template <int MT, int CHG, int CHD, bool HALF>
 int launch_moe(const SkinnyMoeParams& p, bool residual, hipStream_t s, const char* name) {
   constexpr int W = 8, kRows = Shape<HALF>::kRows;
-  skinny_gate_up_kernel<MT, W, CHG, HALF>
-      <<<dim3((unsigned)(p.P / kRows), (unsigned)(p.E + p.shared)), dim3(64 * W), 0, s>>>(p);
+  const dim3 gu((unsigned)(p.P / kRows), (unsigned)(p.E + p.shared));
+  if (HALF && p.norm_w != nullptr)
+    skinny_gate_up_kernel<MT, W, CHG, HALF, HALF><<<gu, dim3(64 * W), 0, s>>>(p);
+  else
+    skinny_gate_up_kernel<MT, W, CHG, HALF><<<gu, dim3(64 * W), 0, s>>>(p);
   if (int rc = check_launch(name)) return rc;
   const dim3 grid((unsigned)(p.H / kRows));
   if (residual)
@@ -447,6 +527,8 @@ bool skinny_fits(int64_t M, int64_t N) {
 
 int skinny_gemm(const SkinnyParams& p, SkinnyEpi epi, hipStream_t s, const char* name) {
   const int cus = device_cu_count();
+  if (p.norm_w != nullptr && (p.M > kNormRows || epi != SkinnyEpi::kF32))
+    return fail(CDX_EUNSUPPORTED, "%s: a folded norm needs M <= 8", name);
   // The columns per block grow with N: one MFMA's worth while that fills the chip at most
   // once, more for wider outputs (fewer blocks and A reads for the same loads in flight).
   if (p.M <= 8) {
@@ -464,8 +546,9 @@ int skinny_gemm(const SkinnyParams& p, SkinnyEpi epi, hipStream_t s, const char*
 
 int skinny_moe(const uint16_t* x, int32_t T, int32_t H, int32_t P, int32_t E, bool shared, const int32_t* perm,
                const int32_t* offsets, const uint16_t* w_gu, const uint16_t* w_down, uint16_t* inter, uint16_t* out,
-               bool residual, hipStream_t s, const char* name) {
-  SkinnyMoeParams p{x, perm, offsets, w_gu, w_down, inter, out, T, H, P, E, shared ? 1 : 0};
+               bool residual, const uint16_t* norm_w, float eps, hipStream_t s, const char* name) {
+  SkinnyMoeParams p{x, perm, offsets, w_gu, w_down, inter, out, T, H, P, E, shared ? 1 : 0, norm_w, eps};
+  if (norm_w != nullptr && T > kNormRows) return fail(CDX_EUNSUPPORTED, "%s: a folded norm needs T <= 8", name);
   if (T <= 8) return launch_moe<1, 4, 4, true>(p, residual, s, name);
   if (T <= 16) return launch_moe<1, 4, 4, false>(p, residual, s, name);
   if (T <= 32) return launch_moe<2, 2, 4, false>(p, residual, s, name);

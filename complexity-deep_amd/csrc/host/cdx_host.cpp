@@ -315,6 +315,90 @@ std::optional<std::tuple<Tensor, OptTensor, OptTensor>> attention(
   return std::make_tuple(out, OptTensor(k), OptTensor(v));
 }
 
+// One decoder block of a generation step (B * S <= 8), h updated in place: the input norm, the
+// attention with its cache, o_proj and its residual add, the post-attention norm, the MoE and
+// its residual add, and mu for the next layer (with mu_w), in six launches: both norms are
+// folded into the products that read them.  Returns (k, v, mu).
+std::optional<std::tuple<Tensor, Tensor, OptTensor>> block_step(
+    const Tensor& h, const Tensor& ln1, double eps1, const OptTensor& mu, const Tensor& w, int64_t nq, int64_t nkv,
+    int64_t D, const OptTensor& qn, const OptTensor& kn, double qk_eps, const Tensor& cos_sin,
+    const OptTensor& past_k, const OptTensor& past_v, const Tensor& o_w, const Tensor& ln2, double eps2,
+    const Tensor& perm, const Tensor& offsets, int64_t E, const Tensor& w_gu, const Tensor& w_down, int64_t ie,
+    bool shared, const OptTensor& mu_w, const OptTensor& mu_param, double mu_lo, double mu_hi, double lo, double hi) {
+  if (!dense(h) || h.dim() != 3 || h.numel() == 0 || !dense(ln1) || !dense(ln2) || !dense(w) || !dense(o_w) ||
+      !dense(w_gu) || !dense(w_down) || w.dim() != 2 || o_w.dim() != 2 || w_gu.dim() != 4 || w_down.dim() != 3)
+    return {};
+  const int64_t B = h.size(0), S = h.size(1), H = h.size(2), M = B * S, N = (nq + 2 * nkv) * D;
+  if (M > 8 || !cdx_few_rows(M, N) || !cdx_few_rows(M, H) || H % 64 != 0 || H > 8192 || ln1.numel() != H ||
+      ln2.numel() != H || nkv <= 0 || nq % nkv != 0 || D <= 0 || D % 8 != 0 || D > 128 || w.size(0) != N ||
+      w.size(1) != 2 * H || o_w.size(0) != H || o_w.size(1) != nq * D || (nq * D) % 64 != 0 || !(eps1 >= 0) ||
+      !(eps2 >= 0) || !(qk_eps >= 0))
+    return {};
+  int64_t ldmu = 0;
+  if (mu) {
+    if (!plain(*mu) || !aligned(*mu) || mu->dim() != 3 || mu->size(0) != B || mu->size(1) != S || mu->size(2) != H)
+      return {};
+    ldmu = row_ld(*mu, H);
+    if (ldmu < 0) return {};
+  }
+  if (qn.has_value() != kn.has_value() || past_k.has_value() != past_v.has_value()) return {};
+  if (qn && (!dense(*qn) || !dense(*kn) || qn->numel() != D || kn->numel() != D)) return {};
+  if (past_k && (!dense(*past_k) || !dense(*past_v) || past_k->dim() != 4 || past_k->size(0) != B ||
+                 past_k->size(1) != nkv || past_k->size(2) == 0 || past_k->size(3) != D ||
+                 past_v->sizes() != past_k->sizes() ||
+                 (at::GradMode::is_enabled() && (past_k->requires_grad() || past_v->requires_grad()))))
+    return {};
+  const int64_t past = past_k ? past_k->size(2) : 0;
+  if (!plain(cos_sin, at::kFloat) || !cos_sin.is_contiguous() || cos_sin.size(0) < past + S ||
+      2 * B * nkv * (past + S) > INT32_MAX / (D / 8))
+    return {};
+  const int64_t P = (ie + 63) / 64 * 64, nb = E + (shared ? 1 : 0);
+  if (!plain(perm, at::kInt) || !plain(offsets, at::kInt) || !perm.is_contiguous() || !offsets.is_contiguous() ||
+      perm.numel() < M || E <= 0 || E > 64 || offsets.numel() < E + 1 || w_gu.size(0) != nb || w_gu.size(1) != 2 ||
+      w_gu.size(2) != P || w_gu.size(3) != H || w_down.size(0) != nb || w_down.size(1) != H || w_down.size(2) != P)
+    return {};
+  if (mu_w && (!mu_param || !dense(*mu_w) || !dense(*mu_param) || mu_w->dim() != 2 || mu_w->size(0) != H ||
+               mu_w->size(1) != H || mu_param->dim() != 1 || mu_param->size(0) != H || !(lo <= hi) || !(mu_lo <= mu_hi)))
+    return {};
+
+  void* st = stream();
+  const float scale = (float)(1.0 / std::sqrt((double)D));
+  const bool attend = S <= 16 && past >= S;
+  Tensor attn = like(h, {B, S, nq * D}), k = like(h, {B, nkv, past + S, D}), v = like(h, {B, nkv, past + S, D});
+  OptTensor q;
+  if (!attend) q = like(h, {B, nq, S, D});
+  const size_t bytes = cdx_qkv_cache_workspace_bytes(B, S, (int32_t)nq, (int32_t)nkv, (int32_t)D);
+  Tensor work = at::empty({(int64_t)bytes}, h.options().dtype(at::kByte).requires_grad(false));
+  check(cdx_qkv_cache_norm_fwd(u16(h), H, u16(ln1), (float)eps1, u16(mu), ldmu, u16(w), u16(w) + H, 2 * H, B, S,
+                               (int32_t)H, (int32_t)nq, (int32_t)nkv, (int32_t)D, u16(qn), u16(kn), (float)qk_eps,
+                               cos_sin.data_ptr<float>(), cos_sin.size(0), u16(past_k), u16(past_v), past,
+                               q ? w16(*q) : nullptr, w16(k), w16(v), attend ? w16(attn) : nullptr, scale,
+                               work.data_ptr(), bytes, st),
+        "cdx_qkv_cache_norm_fwd");
+  if (!attend) {
+    Tensor vt = like(h, {B, nkv, D, 64});  // S <= 8
+    check(cdx_vt_pack(u16(v), B * nkv, past + S, S, (int32_t)D, w16(vt), 64, st), "cdx_vt_pack");
+    check(cdx_attention_cache_fwd(u16(*q), u16(k), u16(vt), B, S, past + S, (int32_t)nq, (int32_t)nkv, (int32_t)D, 64,
+                                  scale, w16(attn), st),
+          "cdx_attention_cache_fwd");
+  }
+  check(cdx_linear_accum_fwd(u16(attn), nq * D, u16(o_w), nq * D, M, (int32_t)(nq * D), (int32_t)H, w16(h), H, st),
+        "cdx_linear_accum_fwd");
+  Tensor inter = like(h, {M, (shared ? 2 : 1) * P});
+  check(cdx_moe_swiglu_norm_residual_fwd(w16(h), u16(ln2), (float)eps2, M, (int32_t)H, (int32_t)ie, (int32_t)E, shared,
+                                         perm.data_ptr<int32_t>(), offsets.data_ptr<int32_t>(), u16(w_gu),
+                                         u16(w_down), w16(inter), st),
+        "cdx_moe_swiglu_norm_residual_fwd");
+  OptTensor mu_out;
+  if (mu_w) {
+    mu_out = like(h, h.sizes());
+    check(cdx_mu_guidance_fwd(u16(h), M, (int32_t)H, u16(*mu_w), u16(*mu_param), (float)mu_lo, (float)mu_hi, (float)lo,
+                              (float)hi, w16(*mu_out), H, st),
+          "cdx_mu_guidance_fwd");
+  }
+  return std::make_tuple(k, v, mu_out);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -328,4 +412,5 @@ PYBIND11_MODULE(_host, m) {
   m.def("route_plans", &route_plans);
   m.def("moe_swiglu", &moe_swiglu);
   m.def("attention", &attention);
+  m.def("block_step", &block_step);
 }

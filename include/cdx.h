@@ -211,6 +211,17 @@ int cdx_moe_swiglu_residual_fwd(const uint16_t* x_dev, int64_t T, int32_t H, int
                                 uint16_t* residual_dev, void* stream);
 
 /*
+ * h[t, :] += MoE(RMSNorm(h))[t, :] in place for T <= 8 tokens (norm weights norm_w [H]): the
+ * norm folded into the gate/up pass as in cdx_qkv_cache_norm_fwd, the add rounded as in
+ * cdx_moe_swiglu_residual_fwd, whose other arguments these are.
+ * Replaces: core/layer.py:176-183 (post_attention_layernorm, mlp and the residual add).
+ */
+int cdx_moe_swiglu_norm_residual_fwd(uint16_t* h_dev, const uint16_t* norm_w_dev, float eps, int64_t T, int32_t H,
+                                     int32_t Ie, int32_t E, int32_t has_shared, const int32_t* perm_dev,
+                                     const int32_t* offsets_dev, const uint16_t* w_gu_dev,
+                                     const uint16_t* w_down_dev, uint16_t* inter_dev, void* stream);
+
+/*
  * Copies expert weights gate, up [E][H][I] and down [E][I][H] ([in, out], the operator API's
  * layout) into the operands above without a shared block: w_gu [E][2][P][H], w_down [E][H][P],
  * units in [I, P) zeroed.  H % 64 == 0, I % 8 == 0, pointers 16-byte aligned.
@@ -359,6 +370,20 @@ int cdx_qkv_cache_fwd(const uint16_t* x_dev, int64_t ldx, const uint16_t* mu_dev
                       const uint16_t* past_k_dev, const uint16_t* past_v_dev, int64_t past, uint16_t* q_out_dev,
                       uint16_t* k_out_dev, uint16_t* v_out_dev, uint16_t* attn_out_dev, float scale, void* work_dev,
                       size_t work_bytes, void* stream);
+
+/*
+ * cdx_qkv_cache_fwd of x = RMSNorm(h) (weights norm_w [H], norm_eps) for B * S <= 8, without
+ * storing x: the product takes bf16(norm_w * h) and its fp32 sums are scaled by 1 / rms(h).
+ * Replaces: core/layer.py:162-173 (input_layernorm and the attention up to o_proj).
+ */
+int cdx_qkv_cache_norm_fwd(const uint16_t* h_dev, int64_t ldh, const uint16_t* norm_w_dev, float norm_eps,
+                           const uint16_t* mu_dev, int64_t ldmu, const uint16_t* w_x_dev, const uint16_t* w_mu_dev,
+                           int64_t ldw, int64_t B, int64_t S, int32_t H, int32_t nq, int32_t nkv, int32_t hd,
+                           const uint16_t* q_norm_w_dev, const uint16_t* k_norm_w_dev, float eps,
+                           const float* cos_sin_dev, int64_t n_pos, const uint16_t* past_k_dev,
+                           const uint16_t* past_v_dev, int64_t past, uint16_t* q_out_dev, uint16_t* k_out_dev,
+                           uint16_t* v_out_dev, uint16_t* attn_out_dev, float scale, void* work_dev,
+                           size_t work_bytes, void* stream);
 
 /*
  * The first S rows of each of `slabs` matrices v [rows][hd] in the transposed layout of
