@@ -48,6 +48,8 @@ _SIGNATURES = {
     "cdx_moe_swiglu_norm_residual_fwd": (ctypes.c_int, [_vp, _vp, ctypes.c_float, _i64, _i32, _i32, _i32, _i32, _vp,
                                                         _vp, _vp, _vp, _vp, _vp]),
     "cdx_moe_pack": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp]),
+    "cdx_cggr_prepare": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "cdx_widen_plan": (ctypes.c_int, [_vp, _i64, _vp, _vp, _i32, _vp, _vp, _vp, _vp]),
     "cdx_grouped_gemm_fwd": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp]),
     "cdx_swiglu_fwd": (ctypes.c_int, [_vp, _vp, _i64, _i32, _i32, _vp, _vp]),
     "cdx_mu_qkv_fwd": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i32, _i32, _vp, _i64,

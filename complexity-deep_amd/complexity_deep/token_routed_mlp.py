@@ -170,6 +170,11 @@ def sort_tokens_by_expert(tokens: torch.Tensor, expert_ids: torch.Tensor, num_ex
     """(sorted_tokens, sorted_indices, expert_offsets [E+1], expert_counts [E]) with int64
     index outputs; cuda/triton_token_routed.py:37-61.  The order inside an expert is the
     original token order (a stable sort)."""
+    fast = nat.host()
+    if fast is not None:
+        done = fast.sort_tokens(tokens, expert_ids, num_experts)
+        if done is not None:
+            return done
     nat.require_device(tokens, expert_ids, dtype=None, what="sort_tokens_by_expert")
     plan = route_plan(expert_ids, None, num_experts)
     rows = tokens.reshape(tokens.shape[0], -1)
@@ -431,6 +436,11 @@ def persistent_swiglu_cggr(sorted_tokens: torch.Tensor, gate_weights: torch.Tens
     ``.data``).  ``num_sms`` is accepted for
     API compatibility."""
     forward_only("persistent_swiglu_cggr", sorted_tokens, gate_weights, up_weights, down_weights)
+    fast = nat.host()
+    if fast is not None and isinstance(expert_offsets, torch.Tensor):
+        done = fast.swiglu_cggr(sorted_tokens, gate_weights, up_weights, down_weights, expert_offsets)
+        if done is not None:
+            return done
     nat.require_device(sorted_tokens, gate_weights, up_weights, down_weights, what="persistent_swiglu_cggr")
     if sorted_tokens.dim() != 2:
         raise ValueError("persistent_swiglu_cggr: sorted_tokens must be [tokens, hidden]")

@@ -228,6 +228,50 @@ OptTensor moe_swiglu(const Tensor& x, const Tensor& perm, const Tensor& offsets,
   return out;
 }
 
+// sort_tokens_by_expert: (rows in expert order, their indices, offsets, counts), indices in 64 bits.
+std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> sort_tokens(const Tensor& tokens, const Tensor& experts,
+                                                                       int64_t E) {
+  const int64_t T = experts.numel();
+  if (!tokens.is_cuda() || !plain(tokens, tokens.scalar_type()) || !tokens.is_contiguous() || !aligned(tokens) ||
+      tokens.dim() < 1 || tokens.size(0) != T || tokens.numel() == 0)
+    return {};
+  auto plan = route_plan(experts, {}, E);
+  if (!plan) return {};
+  const auto& [eid, perm, inv, counts, offsets] = *plan;
+  Tensor rows = like(tokens, tokens.sizes());
+  check(cdx_permute_rows(tokens.data_ptr(), perm.data_ptr<int32_t>(), T, tokens.nbytes() / T, rows.data_ptr(), stream()),
+        "cdx_permute_rows");
+  auto longs = [&](int64_t n) { return at::empty({n}, experts.options()); };
+  Tensor index = longs(T), off64 = longs(E + 1), cnt64 = longs(E);
+  check(cdx_widen_plan(perm.data_ptr<int32_t>(), T, offsets.data_ptr<int32_t>(), counts.data_ptr<int32_t>(), (int32_t)E,
+                       index.data_ptr<int64_t>(), off64.data_ptr<int64_t>(), cnt64.data_ptr<int64_t>(), stream()),
+        "cdx_widen_plan");
+  return std::make_tuple(rows, index, off64, cnt64);
+}
+
+// persistent_swiglu_cggr: pack the weights and prepare the rows in one launch, then both passes.
+OptTensor swiglu_cggr(const Tensor& x, const Tensor& gate, const Tensor& up, const Tensor& down,
+                      const Tensor& offsets) {
+  if (!dense(x) || x.dim() != 2 || x.numel() == 0 || !dense(gate) || !dense(up) || !dense(down) || gate.dim() != 3 ||
+      !plain(offsets, at::kLong) || !offsets.is_contiguous() || offsets.dim() != 1)
+    return {};
+  const int64_t T = x.size(0), H = x.size(1), E = gate.size(0), I = gate.size(2), P = (I + 63) / 64 * 64;
+  if (gate.size(1) != H || up.sizes() != gate.sizes() || down.dim() != 3 || down.size(0) != E || down.size(1) != I ||
+      down.size(2) != H || H % 64 != 0 || I % 8 != 0 || I == 0 || E > 64 || E == 0 || offsets.numel() != E + 1 ||
+      T > INT32_MAX - 256 || T * H * 2 > (int64_t)UINT32_MAX || E * 2 * P * H * 2 > (int64_t)UINT32_MAX)
+    return {};
+  Tensor w_gu = like(x, {E, 2, P, H}), w_down = like(x, {E, H, P}), out = like(x, {T, H}), inter = like(x, {T, P});
+  Tensor off32 = ints(x, {E + 1}), ident = ints(x, {T});
+  void* st = stream();
+  check(cdx_cggr_prepare(u16(gate), u16(up), u16(down), (int32_t)E, (int32_t)H, (int32_t)I, offsets.data_ptr<int64_t>(),
+                         T, w16(w_gu), w16(w_down), off32.data_ptr<int32_t>(), ident.data_ptr<int32_t>(), w16(out), st),
+        "cdx_cggr_prepare");
+  check(cdx_moe_swiglu_fwd(u16(x), T, (int32_t)H, (int32_t)I, (int32_t)E, 0, ident.data_ptr<int32_t>(),
+                           off32.data_ptr<int32_t>(), u16(w_gu), u16(w_down), w16(inter), w16(out), st),
+        "cdx_moe_swiglu_fwd");
+  return out;
+}
+
 // The attention of a call without a mask, up to o_proj: (merged heads [B, S, nq D], k, v),
 // k and v only with a cache.  w is the [N, 2 H] buffer of the projection and mu weights side
 // by side.  past: both or neither.  Covers the fused projection (heads of 32, 64 and 128)
@@ -411,6 +455,8 @@ PYBIND11_MODULE(_host, m) {
   m.def("route_plan", &route_plan);
   m.def("route_plans", &route_plans);
   m.def("moe_swiglu", &moe_swiglu);
+  m.def("sort_tokens", &sort_tokens);
+  m.def("swiglu_cggr", &swiglu_cggr);
   m.def("attention", &attention);
   m.def("block_step", &block_step);
 }

@@ -231,6 +231,23 @@ int cdx_moe_pack(const uint16_t* gate_dev, const uint16_t* up_dev, const uint16_
                  int32_t I, uint16_t* w_gu_dev, uint16_t* w_down_dev, void* stream);
 
 /*
+ * cdx_moe_pack and, in the same launch, what else persistent_swiglu_cggr needs of T sorted
+ * rows: offsets32 = the E + 1 segment offsets clamped to [0, T], ident[i] = i, and zeros in the
+ * rows of out [T, H] outside [offsets[0], offsets[E]).
+ * Replaces: cuda/persistent_cggr.py:479-530 (its arguments' preparation).
+ */
+int cdx_cggr_prepare(const uint16_t* gate_dev, const uint16_t* up_dev, const uint16_t* down_dev, int32_t E, int32_t H,
+                     int32_t I, const int64_t* offsets_dev, int64_t T, uint16_t* w_gu_dev, uint16_t* w_down_dev,
+                     int32_t* offsets32_dev, int32_t* ident_dev, uint16_t* out_dev, void* stream);
+
+/*
+ * perm [T], offsets [E + 1] and counts [E] of a plan as 64-bit integers.
+ * Replaces: cuda/triton_token_routed.py:37-61 (the index type of its results).
+ */
+int cdx_widen_plan(const int32_t* perm_dev, int64_t T, const int32_t* offsets_dev, const int32_t* counts_dev, int32_t E,
+                   int64_t* perm64_dev, int64_t* offsets64_dev, int64_t* counts64_dev, void* stream);
+
+/*
  * Grouped GEMM over expert segments of an already sorted token matrix:
  *   out[offsets[e]:offsets[e+1], :] = a[offsets[e]:offsets[e+1], :] @ W[e]
  * with W given K-contiguous: w_dev is [E][N][K] (W[e] transposed).  K % 64 == 0.

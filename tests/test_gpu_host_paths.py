@@ -102,6 +102,26 @@ def test_operators(cdx):
             bad()
 
 
+@pytest.mark.parametrize("T,H,I,E,offs", [(40, 128, 64, 3, (3, 20, 20, 37)), (700, 256, 72, 2, (0, 300, 700)),
+                                          (513, 320, 200, 4, (100, 100, 256, 400, 512)), (300, 64, 8, 1, (0, 0))])
+def test_expert_operators(cdx, T, H, I, E, offs):
+    print(f"host paths: experts T={T} H={H} I={I} E={E}", flush=True)
+    x = _new(T, H)
+    gate, up, down = (_new(*s, seed=3) * 0.1 for s in ((E, H, I), (E, H, I), (E, I, H)))
+    offsets = torch.tensor(offs, device="cuda")
+    for what, fn in {
+            "cggr": lambda: cdx.persistent_swiglu_cggr(x, gate, up, down, offsets),
+            "cggr int32 offsets": lambda: cdx.persistent_swiglu_cggr(x, gate, up, down, offsets.int()),
+            "cggr strided weights": lambda: cdx.persistent_swiglu_cggr(
+                x, gate.transpose(1, 2).contiguous().transpose(1, 2), up, down, offsets),
+            "cggr strided rows": lambda: cdx.persistent_swiglu_cggr(x.t().contiguous().t(), gate, up, down, offsets)}.items():
+        _same(*_both(fn), what)
+    ids = torch.randint(-1, E + 1, (T,), device="cuda")  # out of range: clamped
+    for t in (x, x[:, :7].contiguous(), x.float(), x.view(T, 2, -1)):
+        for i in (ids, ids.int()):
+            _same(*_both(lambda: cdx.sort_tokens_by_expert(t, i, E)), f"sort {t.dtype} {tuple(t.shape)}")
+
+
 @pytest.mark.parametrize("H,nq,nkv", [(256, 4, 2), (320, 8, 4), (512, 4, 4)])
 def test_attention(cdx, H, nq, nkv):
     print(f"host paths: attention H={H} heads={nq}/{nkv}", flush=True)
