@@ -65,6 +65,9 @@ _SIGNATURES = {
     "cdx_qkv_cache_fwd": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _i32,
                                          _vp, _vp, ctypes.c_float, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp,
                                          ctypes.c_float, _vp, ctypes.c_size_t, _vp]),
+    "cdx_qkv_prompt_fwd": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _i32,
+                                          _vp, _vp, ctypes.c_float, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp,
+                                          ctypes.c_size_t, _vp]),
     "cdx_qkv_cache_norm_fwd": (ctypes.c_int, [_vp, _i64, _vp, ctypes.c_float, _vp, _i64, _vp, _vp, _i64, _i64, _i64,
                                               _i32, _i32, _i32, _i32, _vp, _vp, ctypes.c_float, _vp, _i64, _vp, _vp,
                                               _i64, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, ctypes.c_size_t, _vp]),

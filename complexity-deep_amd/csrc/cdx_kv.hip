@@ -18,7 +18,8 @@
 //                     8 KV heads of 128 (33 MB through the cache) 14.5, of which the
 //                     product 8; 1 sequence of 500, 4 KV heads of 64: 6.7.
 //   vt_pack_kernel    [rows][D] -> V^T tiles in the key order of the attention kernel
-//                     (2 x 777 tokens, 4 heads of 80: 3.6 us).
+//                     (2 x 777 tokens, 4 heads of 80: 3.6 us; a prompt's own V^T is written by
+//                     the pass above instead).
 #include "cdx_gemm.h"
 #include "cdx_skinny.h"
 
@@ -43,7 +44,9 @@ struct QkvCacheParams {
   uint16_t* v;
   uint16_t* attn;  // [B][S][nq D]
   float scale_log2;
-  uint32_t row_blocks;  // blocks of 16 (token, head) rows; the blocks after them copy
+  uint16_t* vt;         // V^T of the new tokens (past == 0), [B][nkv][D][vt_ld], or nullptr
+  int64_t vt_ld;
+  uint32_t row_blocks;  // blocks of 16 (token, head) rows; those after them copy, or write V
 };
 
 // Sum over each row of 16 lanes, returned to all of them.
@@ -68,10 +71,58 @@ __device__ __forceinline__ void store4(uint16_t* p, const float* f) {
   *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]));
 }
 
-template <typename TIn>
+// A staged tile of 64 tokens x D values in LDS (rows of D + 8) to columns s0 .. s0 + 63 of
+// V^T rows (vt_ld apart) in vt_col order: 16-byte writes along the tokens.
+__device__ __forceinline__ void store_vt_tile(const uint16_t* tile, int D, uint16_t* dst, int64_t vt_ld) {
+  const int pitch = D + 8;
+  for (int i = threadIdx.x; i < D * 8; i += 256) {
+    const int d = i >> 3, ck = i & 7;
+    // Columns 8 ck .. 8 ck + 7 hold tokens t .. t + 3 and t + 8 .. t + 11 (vt_col).
+    const uint16_t* p = tile + (16 * (ck >> 1) + 4 * (ck & 1)) * pitch + d;
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int t = (j >> 1) * 8 + (j & 1) * 2;
+      w[j] = (uint32_t)p[t * pitch] | ((uint32_t)p[(t + 1) * pitch] << 16);
+    }
+    *reinterpret_cast<uint4*>(dst + (int64_t)d * vt_ld + ck * 8) = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
+__device__ __forceinline__ uint4 load8_bf16(const float* p) {
+  float f[8];
+  load4(p, f);
+  load4(p + 4, f + 4);
+  return pack8(f);
+}
+__device__ __forceinline__ uint4 load8_bf16(const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); }
+
+// VT: the V heads go by blocks of 64 tokens, which write the cache rows and, through LDS, V^T
+// for the attention kernel (no pass of its own over V).
+template <typename TIn, bool VT>
 __global__ __launch_bounds__(256) void qkv_cache_kernel(const QkvCacheParams p) {
   const int rows_out = p.past + p.S;
-  if (blockIdx.x >= p.row_blocks) {
+  if (VT && blockIdx.x >= p.row_blocks) {
+    __shared__ __attribute__((aligned(16))) uint16_t tile[VT ? 64 * (128 + 8) : 8];
+    const uint32_t vb = blockIdx.x - p.row_blocks, tiles = (p.S + 63) / 64;
+    const uint32_t slab = vb / tiles;
+    const int s0 = (int)(vb - slab * tiles) * 64, b = slab / p.nkv, h = slab - b * p.nkv;
+    const int cpr = p.D / 8, heads = p.nq + 2 * p.nkv;
+    for (int i = threadIdx.x; i < 64 * cpr; i += 256) {
+      const int t = i / cpr, ch = i - t * cpr;
+      uint4 x = make_uint4(0u, 0u, 0u, 0u);
+      if (s0 + t < p.S) {
+        const int64_t m = (int64_t)b * p.S + s0 + t;
+        x = load8_bf16(static_cast<const TIn*>(p.qkv) + (m * heads + p.nq + p.nkv + h) * p.D + ch * 8);
+        *reinterpret_cast<uint4*>(p.v + ((int64_t)slab * rows_out + s0 + t) * p.D + ch * 8) = x;
+      }
+      *reinterpret_cast<uint4*>(tile + t * (p.D + 8) + ch * 8) = x;
+    }
+    __syncthreads();
+    store_vt_tile(tile, p.D, p.vt + (int64_t)slab * p.D * p.vt_ld + s0, p.vt_ld);
+    return;
+  }
+  if (!VT && blockIdx.x >= p.row_blocks) {
     // The old cache: slab (b, kv head) of past * D values moves to slab stride
     // (past + S) * D; K slabs, then V slabs.  (The host bounds the counts to 31 bits.)
     const uint32_t slab = (uint32_t)p.past * p.D / 8, n = slab * p.B * p.nkv;
@@ -93,7 +144,7 @@ __global__ __launch_bounds__(256) void qkv_cache_kernel(const QkvCacheParams p) 
   }
 
   const int g16 = threadIdx.x & 15;
-  const int heads = p.nq + 2 * p.nkv;
+  const int heads = p.nq + (VT ? 1 : 2) * p.nkv;  // heads of a token that go by rows
   const int64_t rows = (int64_t)p.B * p.S * heads;
   const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
   const int half = p.D >> 1;
@@ -115,7 +166,7 @@ __global__ __launch_bounds__(256) void qkv_cache_kernel(const QkvCacheParams p) 
   const bool attend = p.q == nullptr;
   const uint16_t* nw = kind == 1 ? p.k_norm_w : p.q_norm_w;
   const bool norm = nw != nullptr && kind != 2;
-  const TIn* src = static_cast<const TIn*>(p.qkv) + rr * p.D + c;
+  const TIn* src = static_cast<const TIn*>(p.qkv) + (m * (p.nq + 2 * p.nkv) + head) * p.D + c;
   const float* cs = p.cos_sin + ((int64_t)(p.past + s) * half + c) * 2;
   const int64_t base = (b * p.nkv + h / (p.nq / p.nkv)) * p.past * p.D + c;  // the query's old cache slab
   float x1[4], x2[4], t[8], w1[4] = {1.f, 1.f, 1.f, 1.f}, w2[4] = {1.f, 1.f, 1.f, 1.f};
@@ -216,19 +267,7 @@ __global__ __launch_bounds__(256) void vt_pack_kernel(const uint16_t* __restrict
     *reinterpret_cast<uint4*>(tile + t * pitch + ch * 8) = x;
   }
   __syncthreads();
-  uint16_t* dst = vt + (int64_t)blockIdx.y * D * vt_ld + s0;
-  for (int i = threadIdx.x; i < D * 8; i += 256) {
-    const int d = i >> 3, ck = i & 7;
-    // Columns 8 ck .. 8 ck + 7 hold tokens t .. t + 3 and t + 8 .. t + 11 (vt_col).
-    const uint16_t* p = tile + (16 * (ck >> 1) + 4 * (ck & 1)) * pitch + d;
-    uint32_t w[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int t = (j >> 1) * 8 + (j & 1) * 2;
-      w[j] = (uint32_t)p[t * pitch] | ((uint32_t)p[(t + 1) * pitch] << 16);
-    }
-    *reinterpret_cast<uint4*>(dst + (int64_t)d * vt_ld + ck * 8) = make_uint4(w[0], w[1], w[2], w[3]);
-  }
+  store_vt_tile(tile, D, vt + (int64_t)blockIdx.y * D * vt_ld + s0, vt_ld);
 }
 
 }  // namespace
@@ -250,7 +289,8 @@ int qkv_cache(const char* name, const uint16_t* x_norm_w, float x_eps, const uin
               int64_t S, int32_t H, int32_t nq, int32_t nkv, int32_t hd, const uint16_t* q_norm_w,
               const uint16_t* k_norm_w, float eps, const float* cos_sin, int64_t n_pos, const uint16_t* past_k,
               const uint16_t* past_v, int64_t past, uint16_t* q_out, uint16_t* k_out, uint16_t* v_out,
-              uint16_t* attn_out, float scale, void* work, size_t work_bytes, void* stream) {
+              uint16_t* attn_out, float scale, void* work, size_t work_bytes, void* stream, uint16_t* vt = nullptr,
+              int64_t vt_ld = 0) {
   clear_error();
   if (B < 0 || S < 0 || H <= 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || past < 0 || n_pos < 0)
     return fail(CDX_EINVAL, "%s: bad shape B=%lld S=%lld H=%d nq=%d nkv=%d past=%lld", name, (long long)B,
@@ -265,6 +305,8 @@ int qkv_cache(const char* name, const uint16_t* x_norm_w, float x_eps, const uin
     return fail(CDX_EINVAL, "%s: one of q_out and attn_out must be given", name);
   if (attn_out && (S > kAttendRows || past < S))
     return fail(CDX_EUNSUPPORTED, "%s: attn_out needs S <= %d and past >= S", name, kAttendRows);
+  if (vt && (past != 0 || attn_out || vt_ld < S || vt_ld % 64 != 0 || !aligned16(vt)))
+    return fail(CDX_EINVAL, "%s: vt_out needs past == 0, q_out and vt_ld >= S, a multiple of 64", name);
   if (attn_out && !(scale > 0.f)) return fail(CDX_EINVAL, "%s: scale must be > 0", name);
   if (ldx < H || ldw < H || (mu && ldmu != 0 && ldmu < H))
     return fail(CDX_EINVAL, "%s: leading dimension too small", name);
@@ -334,13 +376,23 @@ int qkv_cache(const char* name, const uint16_t* x_norm_w, float x_eps, const uin
   p.v = v_out;
   p.attn = attn_out;
   p.scale_log2 = scale * 1.4426950408889634f;
-  p.row_blocks = (uint32_t)((M * (nq + 2 * nkv) + 15) / 16);
+  p.vt = vt;
+  p.vt_ld = vt_ld;
+  p.row_blocks = (uint32_t)((M * (nq + (vt ? 1 : 2) * nkv) + 15) / 16);
+  if (vt) {
+    const dim3 grid(p.row_blocks + (uint32_t)((S + 63) / 64 * B * nkv));
+    if (few)
+      qkv_cache_kernel<float, true><<<grid, dim3(256), 0, s>>>(p);
+    else
+      qkv_cache_kernel<uint16_t, true><<<grid, dim3(256), 0, s>>>(p);
+    return check_launch(name);
+  }
   const int64_t copies = 2 * B * nkv * past * hd / 8;
   const dim3 grid(p.row_blocks + (uint32_t)((copies + 256 * kCopyVec - 1) / (256 * kCopyVec)));
   if (few)
-    qkv_cache_kernel<float><<<grid, dim3(256), 0, s>>>(p);
+    qkv_cache_kernel<float, false><<<grid, dim3(256), 0, s>>>(p);
   else
-    qkv_cache_kernel<uint16_t><<<grid, dim3(256), 0, s>>>(p);
+    qkv_cache_kernel<uint16_t, false><<<grid, dim3(256), 0, s>>>(p);
   return check_launch(name);
 }
 
@@ -357,6 +409,21 @@ extern "C" int cdx_qkv_cache_fwd(const uint16_t* x, int64_t ldx, const uint16_t*
   return cdx::qkv_cache("cdx_qkv_cache_fwd", nullptr, 0.f, x, ldx, mu, ldmu, w, w_mu, ldw, B, S, H, nq, nkv, hd,
                         q_norm_w, k_norm_w, eps, cos_sin, n_pos, past_k, past_v, past, q_out, k_out, v_out, attn_out,
                         scale, work, work_bytes, stream);
+}
+
+extern "C" int cdx_qkv_prompt_fwd(const uint16_t* x, int64_t ldx, const uint16_t* mu, int64_t ldmu, const uint16_t* w,
+                                  const uint16_t* w_mu, int64_t ldw, int64_t B, int64_t S, int32_t H, int32_t nq,
+                                  int32_t nkv, int32_t hd, const uint16_t* q_norm_w, const uint16_t* k_norm_w,
+                                  float eps, const float* cos_sin, int64_t n_pos, uint16_t* q_out, uint16_t* k_out,
+                                  uint16_t* v_out, uint16_t* vt_out, int64_t vt_ld, void* work, size_t work_bytes,
+                                  void* stream) {
+  using namespace cdx;
+  clear_error();
+  const char* name = "cdx_qkv_prompt_fwd";
+  if (!vt_out) return fail(CDX_EINVAL, "%s: null pointer", name);
+  return qkv_cache(name, nullptr, 0.f, x, ldx, mu, ldmu, w, w_mu, ldw, B, S, H, nq, nkv, hd, q_norm_w, k_norm_w, eps,
+                   cos_sin, n_pos, nullptr, nullptr, 0, q_out, k_out, v_out, nullptr, 1.f, work, work_bytes, stream,
+                   vt_out, vt_ld);
 }
 
 extern "C" int cdx_qkv_cache_norm_fwd(const uint16_t* h, int64_t ldh, const uint16_t* norm_w, float norm_eps,

@@ -344,18 +344,25 @@ std::optional<std::tuple<Tensor, OptTensor, OptTensor>> attention(
   Tensor k = like(x, {B, nkv, P + S, D}), v = like(x, {B, nkv, P + S, D});
   const size_t bytes = cdx_qkv_cache_workspace_bytes(B, S, (int32_t)nq, (int32_t)nkv, (int32_t)D);
   Tensor work = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte).requires_grad(false));
-  check(cdx_qkv_cache_fwd(u16(x), ldx, u16(mu), ldmu, u16(w), w_mu, ldw, B, S, (int32_t)H, (int32_t)nq, (int32_t)nkv,
-                          (int32_t)D, u16(qn), u16(kn), (float)eps, table, n_pos, u16(past_k), u16(past_v), P,
-                          q ? w16(*q) : nullptr, w16(k), w16(v), attend ? w16(out) : nullptr, scale, work.data_ptr(),
-                          bytes, st),
-        "cdx_qkv_cache_fwd");
-  if (!attend) {
-    Tensor vt = like(x, {B, nkv, D, vt_ld});
-    check(cdx_vt_pack(u16(v), B * nkv, P + S, S, (int32_t)D, w16(vt), vt_ld, st), "cdx_vt_pack");
+  Tensor vt;
+  if (!attend) vt = like(x, {B, nkv, D, vt_ld});
+  if (!attend && P == 0) {
+    check(cdx_qkv_prompt_fwd(u16(x), ldx, u16(mu), ldmu, u16(w), w_mu, ldw, B, S, (int32_t)H, (int32_t)nq, (int32_t)nkv,
+                             (int32_t)D, u16(qn), u16(kn), (float)eps, table, n_pos, w16(*q), w16(k), w16(v), w16(vt),
+                             vt_ld, work.data_ptr(), bytes, st),
+          "cdx_qkv_prompt_fwd");
+  } else {
+    check(cdx_qkv_cache_fwd(u16(x), ldx, u16(mu), ldmu, u16(w), w_mu, ldw, B, S, (int32_t)H, (int32_t)nq, (int32_t)nkv,
+                            (int32_t)D, u16(qn), u16(kn), (float)eps, table, n_pos, u16(past_k), u16(past_v), P,
+                            q ? w16(*q) : nullptr, w16(k), w16(v), attend ? w16(out) : nullptr, scale, work.data_ptr(),
+                            bytes, st),
+          "cdx_qkv_cache_fwd");
+    if (!attend) check(cdx_vt_pack(u16(v), B * nkv, P + S, S, (int32_t)D, w16(vt), vt_ld, st), "cdx_vt_pack");
+  }
+  if (!attend)
     check(cdx_attention_cache_fwd(u16(*q), u16(k), u16(vt), B, S, P + S, (int32_t)nq, (int32_t)nkv, (int32_t)D, vt_ld,
                                   scale, w16(out), st),
           "cdx_attention_cache_fwd");
-  }
   return std::make_tuple(out, OptTensor(k), OptTensor(v));
 }
 

@@ -389,6 +389,18 @@ int cdx_qkv_cache_fwd(const uint16_t* x_dev, int64_t ldx, const uint16_t* mu_dev
                       size_t work_bytes, void* stream);
 
 /*
+ * cdx_qkv_cache_fwd of a prompt (no cached tokens), writing V^T for cdx_attention_cache_fwd in
+ * the same pass: vt_out [B, nkv, hd, vt_ld] as cdx_vt_pack of v_out would.
+ * Replaces: core/attention.py:120-161 for heads other than 32, 64 and 128 wide, or few rows.
+ */
+int cdx_qkv_prompt_fwd(const uint16_t* x_dev, int64_t ldx, const uint16_t* mu_dev, int64_t ldmu,
+                       const uint16_t* w_x_dev, const uint16_t* w_mu_dev, int64_t ldw, int64_t B, int64_t S, int32_t H,
+                       int32_t nq, int32_t nkv, int32_t hd, const uint16_t* q_norm_w_dev, const uint16_t* k_norm_w_dev,
+                       float eps, const float* cos_sin_dev, int64_t n_pos, uint16_t* q_out_dev, uint16_t* k_out_dev,
+                       uint16_t* v_out_dev, uint16_t* vt_out_dev, int64_t vt_ld, void* work_dev, size_t work_bytes,
+                       void* stream);
+
+/*
  * cdx_qkv_cache_fwd of x = RMSNorm(h) (weights norm_w [H], norm_eps) for B * S <= 8, without
  * storing x: the product takes bf16(norm_w * h) and its fp32 sums are scaled by 1 / rms(h).
  * Replaces: core/layer.py:162-173 (input_layernorm and the attention up to o_proj).
