@@ -352,17 +352,23 @@ class FusedMuQKVProjection(nn.Module):
                 out[..., self.q_dim + self.kv_dim:])
 
 
+def _as_written(m: nn.Module) -> bool:
+    """Whether calling m runs its class's forward and nothing else: no hook, its own or a
+    global one, and no forward set on the instance."""
+    return not (m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
+                or nn.modules.module._has_any_global_hook())
+
+
 def _plain_norm(m: nn.Module, D: int) -> bool:
     """Whether m is an unhooked nn.RMSNorm over D values with a weight and an eps."""
     return (type(m) is nn.RMSNorm and m.weight is not None and m.weight.shape == (D,) and m.eps is not None
-            and not (m._forward_hooks or m._forward_pre_hooks))
+            and _as_written(m))
 
 
 def _plain_linear(m: nn.Module) -> bool:
     """Whether calling m is exactly F.linear(x, m.weight): no subclass, bias, hook or autocast."""
     return (type(m) is nn.Linear and m.bias is None and type(m.weight) is nn.Parameter
-            and not (m._forward_hooks or m._forward_pre_hooks or torch.is_autocast_enabled()
-                     or nn.modules.module._has_any_global_hook()))
+            and _as_written(m) and not torch.is_autocast_enabled())
 
 
 class QKVWeights:

@@ -20,7 +20,7 @@ import torch.nn.functional as F
 
 from . import _native as nat
 from ._grad import forward_only
-from .attention import ComplexityAttention, _plain_linear
+from .attention import ComplexityAttention, _as_written, _plain_linear
 from .mlp import SwiGLU
 from .normalization import RMSNorm, add_rms_norm, rms_norm
 from .token_routed_mlp import RoutePlan, TokenRoutedMLP
@@ -127,8 +127,7 @@ class TransformerBlock(nn.Module):
         ln = self.post_attention_layernorm
         normed, h = add_rms_norm(attn_out, hidden_states, ln.weight, ln.eps)
         mlp = self.mlp
-        if type(mlp) in (TokenRoutedMLP, SwiGLU) and not (mlp._forward_hooks or mlp._forward_pre_hooks
-                                                          or nn.modules.module._has_any_global_hook()):
+        if type(mlp) in (TokenRoutedMLP, SwiGLU) and _as_written(mlp):
             # h is this call's own tensor: the down pass adds its rows to it, with the
             # roundings of the separate add (one 5 us pass less at 2048 tokens of 768).
             h = self._mlp(normed, token_ids, None, residual=h)
@@ -183,7 +182,7 @@ class TransformerBlock(nn.Module):
         if (fast is None or route is None or type(self).forward_fused is not _FORWARD_FUSED
                 or type(attn) is not ComplexityAttention or type(mlp) is not TokenRoutedMLP
                 or type(ln1) is not RMSNorm or type(ln2) is not RMSNorm or not _plain_linear(attn.o_proj)
-                or attn._forward_hooks or attn._forward_pre_hooks or mlp._forward_hooks or mlp._forward_pre_hooks
+                or "forward_fused" in self.__dict__ or not _as_written(attn) or not _as_written(mlp)
                 or (attn.training and attn.attention_dropout > 0) or not (attn.fused_prologue or attn.other_head_dim)):
             return None
         guide = self.mu_guidance if want_mu else None

@@ -1,0 +1,59 @@
+"""A forward set on a submodule's instance (as dispatch and instrumentation libraries do) is
+called: the block's shorter paths stand aside for it, as they do for hooks."""
+
+import types
+
+import pytest
+import torch
+from torch import nn
+
+import complexity_deep.layer as layer_mod
+from complexity_deep import _native as nat
+from complexity_deep.attention import _plain_linear, _plain_norm
+
+H = 64
+
+
+def _block():
+    return layer_mod.TransformerBlock(H, 128, 2, 1, num_experts=2, vocab_size=32)
+
+
+@pytest.mark.parametrize("name", [None, "self_attn", "mlp", "self_attn.o_proj"])
+def test_generation_step_honours_a_replaced_forward(monkeypatch, name):
+    calls = []
+    monkeypatch.setattr(nat, "host", lambda: types.SimpleNamespace(block_step=lambda *a: calls.append(a)))
+    block = _block().bfloat16()
+    if name is not None:
+        m = block.get_submodule(name)
+        m.forward = m.forward
+    route = types.SimpleNamespace(perm=None, offsets=None, num_experts=2)
+    assert block.step(torch.zeros(1, 1, H, dtype=torch.bfloat16), None, None, route) is None
+    assert len(calls) == (1 if name is None else 0)
+
+
+def test_block_forward_gives_a_replaced_mlp_forward_no_residual(monkeypatch):
+    block = _block()
+    x, seen = torch.ones(1, 2, H), []
+    monkeypatch.setattr(layer_mod, "add_rms_norm", lambda *a: (x, x))
+    block.input_layernorm, block.mu_guidance = nn.Identity(), None
+    block.self_attn.forward = lambda *a, **k: (x, None)
+
+    def mlp(normed, token_ids=None, route=None, residual=None):
+        seen.append(residual)
+        return 2 * normed
+
+    block.mlp.forward = mlp
+    out = block(x)[0]
+    assert seen == [None] and torch.equal(out, 3 * x)
+
+
+def test_predicates_see_instance_forwards_and_global_hooks():
+    lin, norm = nn.Linear(8, 8, bias=False), nn.RMSNorm(8, eps=1e-6)
+    assert _plain_linear(lin) and _plain_norm(norm, 8)
+    handle = nn.modules.module.register_module_forward_pre_hook(lambda m, a: None)
+    try:
+        assert not _plain_linear(lin) and not _plain_norm(norm, 8)
+    finally:
+        handle.remove()
+    lin.forward, norm.forward = lin.forward, norm.forward
+    assert not _plain_linear(lin) and not _plain_norm(norm, 8)
