@@ -252,7 +252,7 @@ def qkv_cache(x: torch.Tensor, mu: Optional[torch.Tensor], w_x: torch.Tensor, w_
     (k, v [B, nkv, past + S, hd]).  For a few queries whose keys are all cached the kernel
     runs the causal attention too and q is None; otherwise attention is None and q is
     [B, nq, S, hd].  past: contiguous (k, v) of [B, nkv, past, hd], or None."""
-    nat.require_device(x, mu, w_x, w_mu, q_norm_w, k_norm_w, *(past or ()), what="qkv_cache")
+    nat.require_device(x, mu, w_x, w_mu, q_norm_w, k_norm_w, *(past or ())[:2], what="qkv_cache")
     B, S, _ = x.shape
     x2, ldx = _rows_view(x, H)
     if ldx == 0:
@@ -264,7 +264,7 @@ def qkv_cache(x: torch.Tensor, mu: Optional[torch.Tensor], w_x: torch.Tensor, w_
     if q_norm_w is not None:
         q_norm_w = q_norm_w.to(x.dtype).contiguous()
         k_norm_w = k_norm_w.to(x.dtype).contiguous()
-    pk, pv = past if past is not None else (None, None)
+    pk, pv = (past[0], past[1]) if past is not None else (None, None)
     P = pk.shape[2] if past is not None else 0
     attend = S <= _ATTEND_ROWS and P >= S
     new = lambda *shape: torch.empty(shape, dtype=x.dtype, device=x.device)  # noqa: E731
@@ -498,7 +498,7 @@ class ComplexityAttention(nn.Module):
         module's shape.  Any other goes through torch.cat and SDPA."""
         if past is None:
             return True
-        k, v = past
+        k, v = past[0], past[1]
         B, S, _ = x.shape
         return (k.dim() == 4 and k.shape == (B, self.num_kv_heads, k.shape[2], self.head_dim) and v.shape == k.shape
                 and k.shape[2] > 0 and 2 * B * self.num_kv_heads * (k.shape[2] + S) * self.head_dim // 8 < 2 ** 31
@@ -567,7 +567,7 @@ class ComplexityAttention(nn.Module):
             fast = nat.host()
             if fast is not None and (fused or self.other_head_dim) and hidden_states.is_cuda:
                 qn = (self.q_norm.weight, self.k_norm.weight) if self.use_qk_norm else (None, None)
-                pk, pv = past_key_value if past_key_value is not None else (None, None)
+                pk, pv = (past_key_value[0], past_key_value[1]) if past_key_value is not None else (None, None)
                 done = fast.attention(hidden_states, mu_prev, self._qkv_w.buffer(self), self.num_heads,
                                       self.num_kv_heads, D, *qn, self.q_norm.eps if self.use_qk_norm else 0.0,
                                       self.rotary_emb.cos_sin_table(past_len + S, hidden_states.device), pk, pv,

@@ -189,7 +189,7 @@ class TransformerBlock(nn.Module):
         if guide is not None and type(guide) is not MuGuidance:
             return None
         qn, kn = (attn.q_norm, attn.k_norm) if attn.use_qk_norm else (None, None)
-        pk, pv = past if past is not None else (None, None)
+        pk, pv = (past[0], past[1]) if past is not None else (None, None)
         n_pos = h.shape[1] + (pk.shape[2] if pk is not None else 0)
         w_gu, w_down = mlp.kernel_weights()
         done = fast.block_step(

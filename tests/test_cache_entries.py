@@ -1,0 +1,21 @@
+"""A cache entry that carries more than (k, v) is read by index, as core/attention.py:157-161
+reads it."""
+
+import types
+
+import torch
+
+import complexity_deep.layer as layer_mod
+from complexity_deep import _native as nat
+
+
+def test_step_and_cache_check_read_the_first_two_of_an_entry(monkeypatch):
+    seen = []
+    monkeypatch.setattr(nat, "host", lambda: types.SimpleNamespace(block_step=lambda *a: seen.append(a[12:14])))
+    block = layer_mod.TransformerBlock(64, 128, 2, 1, num_experts=2, vocab_size=32).bfloat16()
+    k, v = torch.zeros(2, 1, 1, 3, 32, dtype=torch.bfloat16)
+    h = torch.zeros(1, 1, 64, dtype=torch.bfloat16)
+    entry = (k, v, "more")
+    block.step(h, None, entry, types.SimpleNamespace(perm=None, offsets=None, num_experts=2))
+    assert seen[0][0] is k and seen[0][1] is v
+    assert block.self_attn._cache_fits(entry, h)
