@@ -253,13 +253,15 @@ __global__ __launch_bounds__(256) void qkv_cache_kernel(const QkvCacheParams p) 
 
 // V [slabs][rows][D] (tokens 0 .. S - 1 of each slab) to V^T [slabs][D][vt_ld]: a block
 // moves 64 tokens of one slab through LDS, 16-byte reads along D, 16-byte writes along the
-// tokens in vt_col order.  Columns of tokens >= S are cleared.
+// tokens in vt_col order.  Columns of tokens >= S are cleared.  (The slabs are not a grid
+// dimension of their own: y and z end at 65535, which batch x heads may exceed.)
 __global__ __launch_bounds__(256) void vt_pack_kernel(const uint16_t* __restrict__ v, int64_t rows, int S, int D,
                                                       uint16_t* __restrict__ vt, int64_t vt_ld) {
   __shared__ __attribute__((aligned(16))) uint16_t tile[64 * (128 + 8)];
   const int pitch = D + 8, cpr = D / 8;
-  const int s0 = blockIdx.x * 64;
-  const uint16_t* src = v + ((int64_t)blockIdx.y * rows + s0) * D;
+  const uint32_t tiles = ((uint32_t)S + 63) / 64, slab = blockIdx.x / tiles;
+  const int s0 = (int)(blockIdx.x - slab * tiles) * 64;
+  const uint16_t* src = v + ((int64_t)slab * rows + s0) * D;
   for (int i = threadIdx.x; i < 64 * cpr; i += 256) {
     const int t = i / cpr, ch = i - t * cpr;
     uint4 x = make_uint4(0u, 0u, 0u, 0u);
@@ -267,7 +269,7 @@ __global__ __launch_bounds__(256) void vt_pack_kernel(const uint16_t* __restrict
     *reinterpret_cast<uint4*>(tile + t * pitch + ch * 8) = x;
   }
   __syncthreads();
-  store_vt_tile(tile, D, vt + (int64_t)blockIdx.y * D * vt_ld + s0, vt_ld);
+  store_vt_tile(tile, D, vt + (int64_t)slab * D * vt_ld + s0, vt_ld);
 }
 
 }  // namespace
@@ -457,10 +459,11 @@ extern "C" int cdx_vt_pack(const uint16_t* v, int64_t slabs, int64_t rows, int64
   if (vt_ld < S || vt_ld % 64 != 0)
     return fail(CDX_EINVAL, "%s: vt_ld=%lld must be a multiple of 64 that is >= S", name, (long long)vt_ld);
   if (slabs == 0 || S == 0) return CDX_OK;
-  if (slabs > 65535) return fail(CDX_EUNSUPPORTED, "%s: too many slabs (%lld)", name, (long long)slabs);
+  const int64_t tiles = (S + 63) / 64;
+  if (slabs > INT32_MAX / tiles) return fail(CDX_EUNSUPPORTED, "%s: too many slabs (%lld)", name, (long long)slabs);
   if (!v || !vt) return fail(CDX_EINVAL, "%s: null pointer", name);
   if (!aligned16(v) || !aligned16(vt)) return fail(CDX_EUNSUPPORTED, "%s: pointers must be 16-byte aligned", name);
-  vt_pack_kernel<<<dim3((unsigned)((S + 63) / 64), (unsigned)slabs), dim3(256), 0,
-                   reinterpret_cast<hipStream_t>(stream)>>>(v, rows, (int)S, hd, vt, vt_ld);
+  vt_pack_kernel<<<dim3((unsigned)(slabs * tiles)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream)>>>(
+      v, rows, (int)S, hd, vt, vt_ld);
   return check_launch(name);
 }

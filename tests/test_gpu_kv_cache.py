@@ -126,3 +126,16 @@ def test_vt_pack_matches_the_layout(cdx):
         nat.check(nat.lib().cdx_vt_pack(v.data_ptr(), 6, rows, S, D, vt.data_ptr(), vt.shape[-1], nat.stream_of(v)),
                   "cdx_vt_pack")
         assert torch.equal(vt, to_vt_layout(v[:, :, :S].contiguous())), (D, S, rows)
+
+
+def test_vt_pack_of_more_slabs_than_a_grid_axis(cdx):
+    """Batch x KV heads past 65535, the limit of a grid's second axis."""
+    from complexity_deep import _native as nat
+    from complexity_deep.attention import to_vt_layout, vt_ld_for
+    print("vt_pack, 65537 slabs", flush=True)
+    slabs, S, rows, D = 65537, 2, 3, 8
+    v = torch.randn(1, slabs, rows, D, device="cuda").to(bf16)
+    vt = torch.full((1, slabs, D, vt_ld_for(S)), float("nan"), dtype=bf16, device="cuda")
+    nat.check(nat.lib().cdx_vt_pack(v.data_ptr(), slabs, rows, S, D, vt.data_ptr(), vt.shape[-1], nat.stream_of(v)),
+              "cdx_vt_pack")
+    assert torch.equal(vt, to_vt_layout(v[:, :, :S].contiguous()))
