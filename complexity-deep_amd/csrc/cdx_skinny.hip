@@ -383,9 +383,11 @@ __global__ __launch_bounds__(64 * W) void skinny_gate_up_kernel(const SkinnyMoeP
 }
 
 // Down: block = 16 (HALF: 8) output columns; its waves deal out the 64-column K chunks of
-// every weight block in use (the shared one and the experts that have rows).  Rows outside
-// a chunk's segment enter as zeros, so all chunks add into the same accumulators and one
-// bf16 rounding covers shared + routed.
+// every weight block in use (the shared one and the experts that have rows).  All chunks add
+// into the same accumulators, a row outside a chunk's segment keeping the sum it had, so one
+// bf16 rounding covers shared + routed.  (A lane's results are one row's, so the choice is
+// made on them: an operand of zeros in its place would turn an Inf or NaN among one expert's
+// weights into NaNs in every other expert's rows.)
 template <int MT, int W, int CH, bool HALF, bool RESID>
 __global__ __launch_bounds__(64 * W) void skinny_down_kernel(const SkinnyMoeParams p) {
   using Sh = Shape<HALF>;
@@ -465,12 +467,11 @@ __global__ __launch_bounds__(64 * W) void skinny_down_kernel(const SkinnyMoePara
       for (int j = 0; j < MT; ++j) {
         const int pos = j * 16 + r;
         const bool in = pos >= lo[u] && pos < hi[u];
+        f32x4 t = acc[j];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          const uint4 w = __builtin_bit_cast(uint4, xf[u][s][j]);
-          const uint4 z = make_uint4(in ? w.x : 0u, in ? w.y : 0u, in ? w.z : 0u, in ? w.w : 0u);
-          acc[j] = mfma16(wf[u][s], __builtin_bit_cast(bf16x8, z), acc[j]);
-        }
+        for (int s = 0; s < NS; ++s) t = mfma16(wf[u][s], xf[u][s][j], t);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[j][v] = in ? t[v] : acc[j][v];
       }
     }
   }

@@ -86,3 +86,32 @@ def test_segments_that_cover_part_of_the_rows(cdx):
         ref[a:b] = ((torch.nn.functional.silu(t @ g[e].float()) * (t @ u[e].float())) @ d[e].float()).cpu()
     assert_close_bf16(out, ref, "partial segments")
     assert not bool(out[:3].any()) and not bool(out[37:].any())
+
+
+@pytest.mark.parametrize("T", [2, 8, 9, 16, 31, 64])
+@pytest.mark.parametrize("shared", [True, False])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_weights_that_are_not_finite_stay_with_their_expert(cdx, T, shared, bad):
+    """An Inf or NaN in one expert's weights reaches that expert's tokens and no others: their
+    rows have the bits that they have with finite weights."""
+    print(f"few rows, {bad} in one expert, T={T} shared={shared}", flush=True)
+    torch.manual_seed(T)
+    H, E = 256, 4
+    m = cdx.TokenRoutedMLP(H, 96 * E, num_experts=E, vocab_size=500, shared_expert=shared).to(bf16).cuda()
+    ids = torch.arange(T).view(1, T) * 7 % 500
+    ids[0, 1] = 1  # expert 1 has a token
+    ids = ids.cuda()
+    hit = m.token_to_expert[ids[0]] == 1
+    x, r = _data(1, 1, T, H), _data(2, 1, T, H)
+    with torch.no_grad():
+        good = m(x, token_ids=ids)[0]
+        added = m(x, token_ids=ids, residual=r.clone())[0]
+        for name in ("down_proj_w", "gate_proj_w"):
+            w = getattr(m, name).data
+            keep = w[1].clone()
+            w[1] = bad
+            out = m(x, token_ids=ids)[0]
+            out_r = m(x, token_ids=ids, residual=r.clone())[0]
+            w[1] = keep
+            assert bool(hit.any()) and not bool(torch.isfinite(out[hit]).any()), name
+            assert torch.equal(out[~hit], good[~hit]) and torch.equal(out_r[~hit], added[~hit]), name
