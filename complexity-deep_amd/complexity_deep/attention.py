@@ -251,8 +251,10 @@ def qkv_cache(x: torch.Tensor, mu: Optional[torch.Tensor], w_x: torch.Tensor, w_
     RoPE at positions past .. past + S - 1, and the cache with the new rows appended
     (k, v [B, nkv, past + S, hd]).  For a few queries whose keys are all cached the kernel
     runs the causal attention too and q is None; otherwise attention is None and q is
-    [B, nq, S, hd].  past: contiguous (k, v) of [B, nkv, past, hd], or None."""
-    nat.require_device(x, mu, w_x, w_mu, q_norm_w, k_norm_w, *(past or ())[:2], what="qkv_cache")
+    [B, nq, S, hd].  past: contiguous k and v of [B, nkv, past, hd] (its first two items, so
+    also one stacked tensor), or None."""
+    pk, pv = (past[0], past[1]) if past is not None else (None, None)
+    nat.require_device(x, mu, w_x, w_mu, q_norm_w, k_norm_w, pk, pv, what="qkv_cache")
     B, S, _ = x.shape
     x2, ldx = _rows_view(x, H)
     if ldx == 0:
@@ -264,8 +266,7 @@ def qkv_cache(x: torch.Tensor, mu: Optional[torch.Tensor], w_x: torch.Tensor, w_
     if q_norm_w is not None:
         q_norm_w = q_norm_w.to(x.dtype).contiguous()
         k_norm_w = k_norm_w.to(x.dtype).contiguous()
-    pk, pv = (past[0], past[1]) if past is not None else (None, None)
-    P = pk.shape[2] if past is not None else 0
+    P = pk.shape[2] if pk is not None else 0
     attend = S <= _ATTEND_ROWS and P >= S
     new = lambda *shape: torch.empty(shape, dtype=x.dtype, device=x.device)  # noqa: E731
     q = None if attend else new(B, nq, S, hd)

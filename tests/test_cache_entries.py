@@ -3,6 +3,7 @@ reads it."""
 
 import types
 
+import pytest
 import torch
 
 import complexity_deep.layer as layer_mod
@@ -19,3 +20,23 @@ def test_step_and_cache_check_read_the_first_two_of_an_entry(monkeypatch):
     block.step(h, None, entry, types.SimpleNamespace(perm=None, offsets=None, num_experts=2))
     assert seen[0][0] is k and seen[0][1] is v
     assert block.self_attn._cache_fits(entry, h)
+
+
+def test_general_path_reads_a_stacked_entry(monkeypatch):
+    """One [2, B, heads, rows, D] tensor in the place of (k, v): its truth value is never taken."""
+    from complexity_deep import attention
+    seen = []
+
+    class Stop(Exception):
+        pass
+
+    def require(*tensors, **_):
+        seen.extend(tensors)
+        raise Stop
+
+    monkeypatch.setattr(nat, "require_device", require)
+    x, w = torch.zeros(1, 1, 64, dtype=torch.bfloat16), torch.zeros(128, 128, dtype=torch.bfloat16)
+    past = torch.zeros(2, 1, 1, 3, 32, dtype=torch.bfloat16)
+    with pytest.raises(Stop):
+        attention.qkv_cache(x, None, w[:, :64], w[:, 64:], 64, 2, 1, 32, None, None, 0.0, torch.zeros(4, 16, 2), past)
+    assert [t.data_ptr() for t in seen[-2:]] == [past[0].data_ptr(), past[1].data_ptr()]
