@@ -87,6 +87,14 @@ def _weight_sources(w: torch.Tensor, w_mu: Optional[torch.Tensor], mu: Optional[
     return w.data_ptr(), w_mu.data_ptr(), ldw
 
 
+def _check_widths(x: torch.Tensor, mu: Optional[torch.Tensor], H: int, what: str) -> None:
+    """The kernels read rows of H values through the base pointers of x and mu."""
+    if x.shape[-1] != H:
+        raise ValueError(f"{what}: x hidden size {x.shape[-1]} != {H}")
+    if mu is not None and mu.shape[-1] != H:
+        raise ValueError(f"{what}: mu hidden size {mu.shape[-1]} != {H}")
+
+
 def mu_qkv_project(x: torch.Tensor, mu: Optional[torch.Tensor], w_pack: torch.Tensor,
                    H: int, w_mu: Optional[torch.Tensor] = None) -> torch.Tensor:
     """[..., N] = [x | mu] @ [w_x | w_mu]^T (cdx_mu_qkv_fwd).
@@ -94,6 +102,7 @@ def mu_qkv_project(x: torch.Tensor, mu: Optional[torch.Tensor], w_pack: torch.Te
     w_pack is [N, 2H] (x weights then mu weights) or, with ``w_mu`` given, the x
     weights [N, H] alone; with mu=None only its first H columns are read."""
     nat.require_device(x, mu, w_pack, w_mu, what="mu_qkv_project")
+    _check_widths(x, mu, H, "mu_qkv_project")
     lead = x.shape[:-1]
     x2, ldx = _rows_view(x, H)
     if ldx == 0:
@@ -101,8 +110,6 @@ def mu_qkv_project(x: torch.Tensor, mu: Optional[torch.Tensor], w_pack: torch.Te
     M = x.numel() // H
     N = w_pack.shape[0]
     if mu is not None:
-        if mu.shape[-1] != H:
-            raise ValueError(f"mu_qkv_project: mu hidden size {mu.shape[-1]} != {H}")
         mu = mu.expand(*lead, H) if mu.shape[:-1] != lead else mu
         mu2, ldmu = _rows_view(mu, H)
     else:
@@ -153,6 +160,10 @@ def mu_qkv_rope(x: torch.Tensor, mu: Optional[torch.Tensor], w_pack: torch.Tenso
     goes through cdx_mu_qkv_rope_bcast_fwd, which folds its product with W_mu into one
     64-column K block (K = H + 64 instead of 2H)."""
     nat.require_device(x, mu, w_pack, w_mu, q_norm_w, k_norm_w, what="mu_qkv_rope")
+    _check_widths(x, mu, H, "mu_qkv_rope")
+    if w_pack.shape[0] != (nq + 2 * nkv) * hd:
+        raise ValueError(f"mu_qkv_rope: weight has {w_pack.shape[0]} rows, {nq} + 2 x {nkv} heads of {hd} need "
+                         f"{(nq + 2 * nkv) * hd}")
     B, S, _ = x.shape
     x2, ldx = _rows_view(x, H)
     if ldx == 0:
@@ -255,7 +266,11 @@ def qkv_cache(x: torch.Tensor, mu: Optional[torch.Tensor], w_x: torch.Tensor, w_
     also one stacked tensor), or None."""
     pk, pv = (past[0], past[1]) if past is not None else (None, None)
     nat.require_device(x, mu, w_x, w_mu, q_norm_w, k_norm_w, pk, pv, what="qkv_cache")
+    _check_widths(x, mu, H, "qkv_cache")
     B, S, _ = x.shape
+    if w_x.shape[0] != (nq + 2 * nkv) * hd or (pk is not None and not (
+            pk.shape == pv.shape == (B, nkv, pk.shape[2], hd) and pk.is_contiguous() and pv.is_contiguous())):
+        raise ValueError(f"qkv_cache: weight {tuple(w_x.shape)} or cache does not match {nq} + 2 x {nkv} heads of {hd}")
     x2, ldx = _rows_view(x, H)
     if ldx == 0:
         x2, ldx = x.contiguous(), H

@@ -139,3 +139,27 @@ def test_graphed_forward_needs_gpu_eval_model():
         cdx.GraphedForward(m.train(), 1, 8)
     with pytest.raises(ValueError, match="needs a GPU model"):
         cdx.GraphedForward(m.eval(), 1, 8)
+
+
+@pytest.mark.parametrize("what", ["mu_qkv_project", "mu_qkv_rope", "qkv_cache"])
+@pytest.mark.parametrize("x_shape,mu_shape", [((1, 4, 64), (1, 4, 32)), ((1, 4, 64), (1, 4, 128)),
+                                              ((1, 4, 64), (1, 1, 32)), ((1, 4, 32), (1, 4, 64)),
+                                              ((1, 4, 128), None)])
+def test_operand_widths_are_checked_before_any_launch(monkeypatch, what, x_shape, mu_shape):
+    """The kernels read B * S rows of H values through the base pointers: an x or mu of another
+    width raises on the host."""
+    from complexity_deep import _native as nat
+    from complexity_deep import attention
+    monkeypatch.setattr(nat, "require_device", lambda *a, **k: None)
+    monkeypatch.setattr(nat, "lib", lambda: pytest.fail("reached the library"))
+    x = torch.zeros(x_shape, dtype=torch.bfloat16)
+    mu = None if mu_shape is None else torch.zeros(mu_shape, dtype=torch.bfloat16)
+    w = torch.zeros(128, 128, dtype=torch.bfloat16)
+    table = torch.zeros(4, 16, 2)
+    with pytest.raises((ValueError, RuntimeError), match="hidden|expand"):
+        if what == "mu_qkv_project":
+            attention.mu_qkv_project(x, mu, w, 64)
+        elif what == "mu_qkv_rope":
+            attention.mu_qkv_rope(x, mu, w, 64, 2, 1, 32, None, None, 0.0, table)
+        else:
+            attention.qkv_cache(x, mu, w[:, :64], w[:, 64:], 64, 2, 1, 32, None, None, 0.0, table)
