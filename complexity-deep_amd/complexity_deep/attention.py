@@ -554,10 +554,12 @@ class ComplexityAttention(nn.Module):
         the model keeps it.  The few rows of a generation step run on the kernels for few
         rows instead (4 x 2048 x 2048: 4.4 us, the library's 8.4 us), unless o_proj is
         more than a plain Linear."""
-        w = self.o_proj.weight
-        own = (few_rows(attn.shape[0] * attn.shape[1], w.shape[0]) and _plain_linear(self.o_proj)
-               and w.dtype == attn.dtype and w.is_contiguous() and w.data_ptr() % 16 == 0
-               and w.shape[0] % 8 == 0 and w.shape[1] % 64 == 0)
+        rows = attn.shape[0] * attn.shape[1]
+        own = rows <= 64 and _plain_linear(self.o_proj)
+        if own:
+            w = self.o_proj.weight
+            own = (few_rows(rows, w.shape[0]) and w.dtype == attn.dtype and w.is_contiguous()
+                   and w.data_ptr() % 16 == 0 and w.shape[0] % 8 == 0 and w.shape[1] % 64 == 0)
         if residual is None:
             return linear(attn, w) if own else self.o_proj(attn)
         if residual.shape[:-1] != attn.shape[:-1] or not residual.is_contiguous():

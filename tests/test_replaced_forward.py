@@ -57,3 +57,11 @@ def test_predicates_see_instance_forwards_and_global_hooks():
         handle.remove()
     lin.forward, norm.forward = lin.forward, norm.forward
     assert not _plain_linear(lin) and not _plain_norm(norm, 8)
+
+
+def test_an_output_projection_without_a_weight_of_its_own_is_called():
+    attn = _block().self_attn
+    inner = attn.o_proj
+    attn.o_proj = nn.Sequential(inner, nn.Dropout(0.0))
+    x = torch.randn(1, 2, H)
+    assert torch.equal(attn._out_proj(x, None), inner(x))
