@@ -31,6 +31,7 @@ of more than a few rows a library GEMM.
 
 from __future__ import annotations
 
+import sys
 from typing import Optional, Tuple
 
 import torch
@@ -368,11 +369,33 @@ class FusedMuQKVProjection(nn.Module):
                 out[..., self.q_dim + self.kv_dim:])
 
 
+# The methods that the shorter paths stand in for, as the modules of their classes define them:
+# dispatch and instrumentation libraries replace them, on the instance or on the class (then
+# also before this import, which is why a method of another module's is not taken down).
+_WRITTEN: dict = {}
+
+
+def _own_method(cls: type, name: str):
+    f = getattr(cls, name)
+    return f if getattr(f, "__globals__", None) is vars(sys.modules[cls.__module__]) else None
+
+
+def _written(*classes: type) -> None:
+    _WRITTEN.update({c: _own_method(c, "forward") for c in classes})
+
+
+_MODULE_CALL = _own_method(nn.Module, "__call__")
+_written(nn.Linear, nn.RMSNorm)
+
+
 def _as_written(m: nn.Module) -> bool:
-    """Whether calling m runs its class's forward and nothing else: no hook, its own or a
-    global one, and no forward set on the instance."""
-    return not (m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
-                or nn.modules.module._has_any_global_hook())
+    """Whether calling m runs the forward its class was written with and nothing else: no hook,
+    its own or a global one, and no forward set on the instance or the class.  (Of the classes
+    given to _written; False for any other.)"""
+    cls = type(m)
+    return (cls.forward is _WRITTEN.get(cls) and cls.__call__ is _MODULE_CALL
+            and not (m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
+                     or nn.modules.module._has_any_global_hook()))
 
 
 def _plain_norm(m: nn.Module, D: int) -> bool:
@@ -646,6 +669,7 @@ class ComplexityAttention(nn.Module):
 
 
 MuGuidedAttention = ComplexityAttention
+_written(ComplexityAttention)
 
 __all__ = ["ComplexityAttention", "MuGuidedAttention", "FusedMuQKVProjection", "fused_mu_qkv_projection",
            "mu_qkv_project", "mu_qkv_rope", "causal_attention", "to_vt_layout", "vt_columns", "QKVWeights"]

@@ -20,10 +20,12 @@ import torch.nn.functional as F
 
 from . import _native as nat
 from ._grad import forward_only
-from .attention import ComplexityAttention, _as_written, _plain_linear
+from .attention import ComplexityAttention, _as_written, _plain_linear, _written
 from .mlp import SwiGLU
 from .normalization import RMSNorm, add_rms_norm, rms_norm
 from .token_routed_mlp import RoutePlan, TokenRoutedMLP
+
+_written(TokenRoutedMLP, SwiGLU)
 
 
 def mu_guidance(h: torch.Tensor, w: torch.Tensor, mu: torch.Tensor, mu_lo: float = -math.inf,
@@ -174,19 +176,22 @@ class TransformerBlock(nn.Module):
         """One block of a generation step of at most 8 rows, h updated in place: what
         forward_fused computes without a mask, with both norms folded into the products
         that read them.  Returns (new_kv, mu), or None, nothing having run, if the block is
-        not the plain one (a replaced or hooked submodule, a dense MLP) or the operands are
-        not the usual ones."""
+        not the plain one (a replaced or hooked submodule or method, a dense MLP) or the
+        operands are not the usual ones."""
         fast = nat.host()
         attn, mlp = self.self_attn, self.mlp
         ln1, ln2 = self.input_layernorm, self.post_attention_layernorm
-        if (fast is None or route is None or type(self).forward_fused is not _FORWARD_FUSED
+        cls, own = type(self), self.__dict__
+        if (fast is None or route is None or cls.forward_fused is not _FORWARD_FUSED or cls._mlp is not _MLP
+                or "forward_fused" in own or "_mlp" in own
                 or type(attn) is not ComplexityAttention or type(mlp) is not TokenRoutedMLP
                 or type(ln1) is not RMSNorm or type(ln2) is not RMSNorm or not _plain_linear(attn.o_proj)
-                or "forward_fused" in self.__dict__ or not _as_written(attn) or not _as_written(mlp)
+                or not _as_written(attn) or not _as_written(mlp)
                 or (attn.training and attn.attention_dropout > 0) or not (attn.fused_prologue or attn.other_head_dim)):
             return None
         guide = self.mu_guidance if want_mu else None
-        if guide is not None and type(guide) is not MuGuidance:
+        if guide is not None and (type(guide) is not MuGuidance or MuGuidance.fused is not _FUSED
+                                  or "fused" in guide.__dict__):
             return None
         qn, kn = (attn.q_norm, attn.k_norm) if attn.use_qk_norm else (None, None)
         pk, pv = (past[0], past[1]) if past is not None else (None, None)
@@ -205,4 +210,5 @@ class TransformerBlock(nn.Module):
         return (k, v), mu
 
 
-_FORWARD_FUSED = TransformerBlock.forward_fused
+# What TransformerBlock.step stands in for, as written above.
+_FORWARD_FUSED, _MLP, _FUSED = TransformerBlock.forward_fused, TransformerBlock._mlp, MuGuidance.fused

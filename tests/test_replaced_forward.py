@@ -1,5 +1,5 @@
-"""A forward set on a submodule's instance (as dispatch and instrumentation libraries do) is
-called: the block's shorter paths stand aside for it, as they do for hooks."""
+"""A forward set on a submodule's instance or class (as dispatch and instrumentation libraries
+do) is called: the block's shorter paths stand aside for it, as they do for hooks."""
 
 import types
 
@@ -65,3 +65,41 @@ def test_an_output_projection_without_a_weight_of_its_own_is_called():
     attn.o_proj = nn.Sequential(inner, nn.Dropout(0.0))
     x = torch.randn(1, 2, H)
     assert torch.equal(attn._out_proj(x, None), inner(x))
+
+
+def _step_calls(monkeypatch, block):
+    """How often a step of the block reaches the native block_step."""
+    calls = []
+    monkeypatch.setattr(nat, "host", lambda: types.SimpleNamespace(block_step=lambda *a: calls.append(a)))
+    route = types.SimpleNamespace(perm=None, offsets=None, num_experts=2)
+    assert block.step(torch.zeros(1, 1, H, dtype=torch.bfloat16), None, None, route) is None
+    return len(calls)
+
+
+@pytest.mark.parametrize("cls,name", [
+    (None, None), (layer_mod.ComplexityAttention, "forward"), (layer_mod.TokenRoutedMLP, "forward"),
+    (layer_mod.MuGuidance, "fused"), (layer_mod.TransformerBlock, "_mlp"), (nn.Linear, "forward"),
+    (nn.Module, "__call__")])
+def test_generation_step_honours_a_method_replaced_on_its_class(monkeypatch, cls, name):
+    block = _block().bfloat16()
+    if cls is not None:
+        own = getattr(cls, name)
+        monkeypatch.setattr(cls, name, lambda self, *a, **k: own(self, *a, **k))
+    assert _step_calls(monkeypatch, block) == (1 if cls is None else 0)
+
+
+@pytest.mark.parametrize("path,name", [("", "_mlp"), ("", "forward_fused"), ("mu_guidance", "fused")])
+def test_generation_step_honours_a_method_replaced_on_an_instance(monkeypatch, path, name):
+    block = _block().bfloat16()
+    m = block.get_submodule(path)
+    setattr(m, name, getattr(m, name))
+    assert _step_calls(monkeypatch, block) == 0
+
+
+def test_predicates_see_class_forwards(monkeypatch):
+    lin, norm = nn.Linear(8, 8, bias=False), nn.RMSNorm(8, eps=1e-6)
+    assert _plain_linear(lin) and _plain_norm(norm, 8)
+    for m in (lin, norm):
+        own = type(m).forward
+        monkeypatch.setattr(type(m), "forward", lambda self, x, own=own: own(self, x))
+    assert not _plain_linear(lin) and not _plain_norm(norm, 8)
