@@ -235,7 +235,8 @@ class ComplexityModel(nn.Module):
         for i, layer in enumerate(layers):
             last = i + 1 == n_layers
             past = past_key_values[i] if past_key_values is not None else None
-            done = layer.step(h, mu_prev, past, plans[i], want_mu=not last) if steps else None
+            step = getattr(layer, "step", None) if steps else None  # (a replaced layer may have none)
+            done = step(h, mu_prev, past, plans[i], want_mu=not last) if step is not None else None
             if done is not None:
                 new_kv, mu = done
                 normed = None

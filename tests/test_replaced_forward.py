@@ -103,3 +103,29 @@ def test_predicates_see_class_forwards(monkeypatch):
         own = type(m).forward
         monkeypatch.setattr(type(m), "forward", lambda self, x, own=own: own(self, x))
     assert not _plain_linear(lin) and not _plain_norm(norm, 8)
+
+
+def test_a_layer_that_provides_forward_fused_alone(monkeypatch):
+    """An object with forward_fused and no step in a layer's place serves calls of few rows too."""
+    import complexity_deep.modeling as modeling
+
+    class Layer(nn.Module):
+        use_token_routed_mlp = False
+
+        def __init__(self):
+            super().__init__()
+            self.input_layernorm = nn.LayerNorm(H)
+
+        def forward_fused(self, h, normed, next_norm, **kw):
+            return h + 1, normed + 1, None, None
+
+    model = modeling.ComplexityModel(modeling.ComplexityConfig(
+        vocab_size=32, hidden_size=H, intermediate_size=128, num_hidden_layers=2, num_attention_heads=2,
+        num_key_value_heads=1, num_experts=2))
+    model.layers = nn.ModuleList([Layer(), Layer()])
+    monkeypatch.setattr(modeling, "embedding", lambda ids, w: torch.zeros(*ids.shape, H))
+    monkeypatch.setattr(modeling, "rms_norm", lambda h, w, eps: h)
+    monkeypatch.setattr(modeling, "linear", lambda x, w: x)
+    with torch.no_grad():
+        out = model(torch.zeros(1, 1, dtype=torch.long))
+    assert torch.equal(out.logits, torch.full((1, 1, H), 2.0))
