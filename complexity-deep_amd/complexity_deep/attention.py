@@ -385,7 +385,7 @@ def _written(*classes: type) -> None:
 
 
 _MODULE_CALL = _own_method(nn.Module, "__call__")
-_written(nn.Linear, nn.RMSNorm)
+_written(nn.Linear, nn.RMSNorm, RotaryEmbedding)
 
 
 def _as_written(m: nn.Module) -> bool:
@@ -528,7 +528,7 @@ class ComplexityAttention(nn.Module):
         norms and rotary tables in place."""
         D = self.head_dim
         return (D not in (32, 64, 128) and D % 8 == 0 and D <= 128 and self.hidden_size % 64 == 0
-                and type(self.rotary_emb) is RotaryEmbedding
+                and type(self.rotary_emb) is RotaryEmbedding and _as_written(self.rotary_emb)
                 and (not self.use_qk_norm or (_plain_norm(self.q_norm, D) and _plain_norm(self.k_norm, D)
                                               and self.q_norm.eps == self.k_norm.eps)))
 

@@ -129,3 +129,31 @@ def test_a_layer_that_provides_forward_fused_alone(monkeypatch):
     with torch.no_grad():
         out = model(torch.zeros(1, 1, dtype=torch.long))
     assert torch.equal(out.logits, torch.full((1, 1, H), 2.0))
+
+
+def _hook(m):
+    m.register_forward_hook(lambda *a: None)
+
+
+def _own_forward(m):
+    m.forward = m.forward
+
+
+@pytest.mark.parametrize("change", [None, _hook, _own_forward])
+@pytest.mark.parametrize("name", ["q_norm", "k_norm", "rotary_emb"])
+def test_heads_of_other_dims_honour_a_replaced_norm_or_rotary_forward(change, name):
+    """Heads of 40 took their norms and rotary tables through the submodules' forwards: the
+    kernels stand in for them only where those are as written."""
+    attn = layer_mod.ComplexityAttention(320, 8, 4)
+    assert attn.other_head_dim
+    if change is not None:
+        change(getattr(attn, name))
+        assert not attn.other_head_dim
+
+
+def test_heads_of_other_dims_honour_a_rotary_forward_replaced_on_the_class(monkeypatch):
+    attn = layer_mod.ComplexityAttention(320, 8, 4)
+    cls = type(attn.rotary_emb)
+    own = cls.forward
+    monkeypatch.setattr(cls, "forward", lambda self, n: own(self, n))
+    assert not attn.other_head_dim
