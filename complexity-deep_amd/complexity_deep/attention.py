@@ -533,14 +533,18 @@ class ComplexityAttention(nn.Module):
                                               and self.q_norm.eps == self.k_norm.eps)))
 
     def _cache_fits(self, past, x: torch.Tensor) -> bool:
-        """Whether the kernels take this KV cache (None does): plain contiguous tensors of the
-        module's shape.  Any other goes through torch.cat and SDPA."""
+        """Whether the kernels take this KV cache (None: a prompt): plain contiguous tensors of
+        the module's shape, and counts within cdx_qkv_cache_fwd's 31 bits (16-byte pieces of
+        the caches, (token, head) rows).  Any other goes through torch.cat and SDPA."""
+        B, S, _ = x.shape
+        D, nq, nkv = self.head_dim, self.num_heads, self.num_kv_heads
+        rows = S + (past[0].shape[2] if past is not None else 0)
+        if 2 * B * nkv * rows * D // 8 >= 2 ** 31 or B * S * (nq + 2 * nkv) >= 2 ** 31:
+            return False
         if past is None:
             return True
         k, v = past[0], past[1]
-        B, S, _ = x.shape
-        return (k.dim() == 4 and k.shape == (B, self.num_kv_heads, k.shape[2], self.head_dim) and v.shape == k.shape
-                and k.shape[2] > 0 and 2 * B * self.num_kv_heads * (k.shape[2] + S) * self.head_dim // 8 < 2 ** 31
+        return (k.dim() == 4 and k.shape == (B, nkv, k.shape[2], D) and v.shape == k.shape and k.shape[2] > 0
                 and all(t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
                         and not (t.requires_grad and torch.is_grad_enabled()) for t in (k, v)))
 

@@ -336,7 +336,7 @@ std::optional<std::tuple<Tensor, OptTensor, OptTensor>> attention(
                  past_k->size(1) != nkv || past_k->size(3) != D || past_v->sizes() != past_k->sizes() || P == 0 ||
                  (at::GradMode::is_enabled() && (past_k->requires_grad() || past_v->requires_grad()))))
     return {};
-  if (2 * B * nkv * (P + S) > INT32_MAX / (D / 8)) return {};
+  if (2 * B * nkv * (P + S) > INT32_MAX / (D / 8) || M > INT32_MAX / (nq + 2 * nkv)) return {};
   const bool attend = S <= 16 && P >= S;
   OptTensor q;
   if (!attend) q = like(x, {B, nq, S, D});

@@ -40,3 +40,20 @@ def test_general_path_reads_a_stacked_entry(monkeypatch):
     with pytest.raises(Stop):
         attention.qkv_cache(x, None, w[:, :64], w[:, 64:], 64, 2, 1, 32, None, None, 0.0, torch.zeros(4, 16, 2), past)
     assert [t.data_ptr() for t in seen[-2:]] == [past[0].data_ptr(), past[1].data_ptr()]
+
+
+def test_calls_past_the_kernels_counts_keep_the_torch_path():
+    """cdx_qkv_cache_fwd counts the cache's 16-byte pieces, and (token, head) rows, in 31 bits:
+    a prompt beyond that, with or without a cache, is not given to it."""
+    from complexity_deep.attention import ComplexityAttention
+    with torch.device("meta"):
+        attn = ComplexityAttention(320, 8, 4).bfloat16()
+        few_kv = ComplexityAttention(1024, 128, 1).bfloat16()
+
+    def fits(m, tokens, past=None):
+        return m._cache_fits(past, torch.empty(1, tokens, m.hidden_size, dtype=torch.bfloat16, device="meta"))
+
+    edge = 2 ** 31 // (2 * 4 * 5)  # 2 x 4 KV heads of 40, five pieces each
+    assert fits(attn, edge) and not fits(attn, edge + 1)
+    rows = 2 ** 31 // 130
+    assert fits(few_kv, rows) and not fits(few_kv, rows + 1)
