@@ -132,7 +132,8 @@ OptTensor linear(const Tensor& x, const Tensor& w) {
 bool linear_accumulate(const Tensor& x, const Tensor& w, const Tensor& residual) {
   if (!dense(x) || !dense(w) || !dense(residual) || w.dim() != 2 || x.dim() < 2 || x.numel() == 0) return false;
   const int64_t N = w.size(0), K = w.size(1);
-  if (x.size(-1) != K || residual.size(-1) != N || residual.numel() / N != x.numel() / K || K % 64 != 0 || N % 8 != 0 ||
+  if (x.size(-1) != K || residual.dim() != x.dim() || residual.size(-1) != N ||
+      residual.sizes().slice(0, x.dim() - 1) != x.sizes().slice(0, x.dim() - 1) || K % 64 != 0 || N % 8 != 0 || N == 0 ||
       N > INT32_MAX || K > INT32_MAX)
     return false;
   const int64_t M = x.numel() / K;
@@ -282,7 +283,8 @@ std::optional<std::tuple<Tensor, OptTensor, OptTensor>> attention(
     bool use_cache) {
   if (!plain(x) || !aligned(x) || x.dim() != 3 || x.numel() == 0 || !dense(w) || w.dim() != 2) return {};
   const int64_t B = x.size(0), S = x.size(1), H = x.size(2), M = B * S, N = (nq + 2 * nkv) * D;
-  if (H % 64 != 0 || w.size(0) != N || w.size(1) != 2 * H || nkv <= 0 || nq % nkv != 0 || D % 8 != 0 || D > 128)
+  if (H % 64 != 0 || w.size(0) != N || w.size(1) != 2 * H || nkv <= 0 || nq % nkv != 0 || D <= 0 || D % 8 != 0 ||
+      D > 128)
     return {};
   const int64_t ldx = row_ld(x, H);
   if (ldx < H) return {};

@@ -201,3 +201,20 @@ def test_block_step(cdx, oracle, H, I, nq, nkv, E, B, S, past):
             _near(x, y, f"{what}, scale {scale}")
     blk.self_attn.register_forward_hook(lambda *a: None)
     assert blk.step(h.clone(), mu, kv, plan) is None  # a hook is not passed by
+
+
+def test_linear_accumulate_checks_every_size(cdx):
+    """A weight without rows, and a residual of the right row count but other leading sizes, raise
+    on both paths."""
+    from complexity_deep import _native as nat
+    from complexity_deep.linear import linear_accumulate_
+    print("host paths: linear_accumulate_ sizes", flush=True)
+    x, w = _new(2, 3, 128), _new(64, 128)
+    for res, weight in ((_new(2, 3, 64)[..., :0], w[:0]), (_new(6, 64), w), (_new(2, 64), w), (_new(2, 3, 56), w)):
+        for hook in (None, lambda *a: None):
+            nat.set_launch_hook(hook)
+            try:
+                with pytest.raises((ValueError, RuntimeError)), torch.no_grad():
+                    linear_accumulate_(x, weight, res)
+            finally:
+                nat.set_launch_hook(None)
