@@ -50,8 +50,9 @@ def _rows_view(t: torch.Tensor, H: int) -> Tuple[torch.Tensor, int]:
     if t.shape[-1] == H and t.is_contiguous():
         return t, H
     if t.stride(-1) != 1:
-        t = t.contiguous()
-    if t.dim() > 1 and all(s == 0 for s in t.stride()[:-1]):
+        return t.contiguous(), H
+    # (Dimensions of size 1 have no say: expand() leaves them any stride.)
+    if t.dim() > 1 and all(s == 0 for n, s in zip(t.shape[:-1], t.stride()[:-1]) if n != 1):
         return t, 0
     try:
         rows = t.view(-1, H)

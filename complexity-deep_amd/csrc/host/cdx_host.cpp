@@ -54,15 +54,15 @@ inline Tensor ints(const Tensor& t, at::IntArrayRef shape) {
 }
 
 // Row stride of a [..., H] view whose rows are evenly spaced with unit stride inside (0: one
-// row for all), or -1.
+// row for all), or -1.  Dimensions of size 1 have no say: expand() leaves them any stride.
 int64_t row_ld(const Tensor& t, int64_t H) {
   if (t.dim() < 1 || t.size(-1) != H || t.stride(-1) != 1) return -1;
   if (t.is_contiguous()) return H;
   int64_t ld = -1, next = 0;
   bool bcast = t.dim() > 1;
   for (int64_t d = t.dim() - 2; d >= 0; --d) {
-    if (t.stride(d) != 0) bcast = false;
     if (t.size(d) == 1) continue;
+    if (t.stride(d) != 0) bcast = false;
     if (ld < 0)
       ld = t.stride(d);
     else if (t.stride(d) != next)

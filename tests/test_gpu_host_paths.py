@@ -203,6 +203,31 @@ def test_block_step(cdx, oracle, H, I, nq, nkv, E, B, S, past):
     assert blk.step(h.clone(), mu, kv, plan) is None  # a hook is not passed by
 
 
+@pytest.mark.parametrize("H,nq,nkv", [(256, 4, 2), (320, 8, 4)])
+def test_one_mu_row_for_every_token_takes_the_native_paths(cdx, H, nq, nkv):
+    """mu of [1, 1, H] expanded to the batch (a model's first layer) is one broadcast row
+    whatever the sizes are: expand() keeps the old stride in dimensions of size 1."""
+    from complexity_deep import _native as nat
+    print(f"host paths: one mu row, H={H}", flush=True)
+    torch.manual_seed(H)
+    blk = cdx.TransformerBlock(H, 704, nq, nkv, num_experts=4, vocab_size=500).to(bf16).cuda().eval()
+    m, row = blk.self_attn, _new(1, 1, H)
+    norms = (m.q_norm.weight, m.k_norm.weight, m.q_norm.eps)
+    for B, S in ((4, 1), (1, 4), (2, 3), (1, 150), (3, 50)):
+        x, mu = _new(B, S, H), row.expand(B, S, H)
+        with torch.no_grad():
+            table = m.rotary_emb.cos_sin_table(S, x.device)
+            assert nat.host().attention(x, mu, m._qkv_w.buffer(m), nq, nkv, H // nq, *norms, table, None, None,
+                                        True if B * S <= 8 else False) is not None, (B, S)
+            if B * S <= 8:
+                plan = blk.mlp.plan(torch.zeros(B, S, dtype=torch.long, device="cuda"))
+                assert blk.step(x.clone(), mu, None, plan) is not None, (B, S)
+            a, b = _both(lambda: m(x, mu_prev=mu)[0])
+            c = m(x, mu_prev=mu.contiguous())[0]
+        _same(a, b, (B, S))
+        _near(a, c, (B, S))
+
+
 def test_linear_accumulate_checks_every_size(cdx):
     """A weight without rows, and a residual of the right row count but other leading sizes, raise
     on both paths."""

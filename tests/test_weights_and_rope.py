@@ -163,3 +163,16 @@ def test_operand_widths_are_checked_before_any_launch(monkeypatch, what, x_shape
             attention.mu_qkv_rope(x, mu, w, 64, 2, 1, 32, None, None, 0.0, table)
         else:
             attention.qkv_cache(x, mu, w[:, :64], w[:, 64:], 64, 2, 1, 32, None, None, 0.0, table)
+
+
+@pytest.mark.parametrize("B,S", [(4, 1), (1, 4), (3, 5), (1, 1)])
+def test_an_expanded_row_is_one_row(B, S):
+    """[1, 1, H] expanded to the batch: stride 0 in every dimension that has more than one entry
+    (one token: a contiguous row), without a copy."""
+    from complexity_deep.attention import _rows_view
+    row = torch.zeros(1, 1, 64)
+    t, ld = _rows_view(row.expand(B, S, 64), 64)
+    assert ld == (0 if B * S > 1 else 64) and t.data_ptr() == row.data_ptr()
+    assert _rows_view(torch.zeros(2, 1, 64).expand(2, 3, 64), 64)[1] == 64  # a row per sequence
+    assert _rows_view(torch.zeros(1, 2, 64).expand(3, 2, 64), 64)[1] == 64  # a row per position
+    assert _rows_view(torch.zeros(1, 1, 128)[..., ::2], 64)[1] == 64
