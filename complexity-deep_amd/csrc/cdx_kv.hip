@@ -232,8 +232,11 @@ __global__ __launch_bounds__(256) void qkv_cache_kernel(const QkvCacheParams p) 
 #pragma unroll
     for (int i = 0; i < 4; ++i) dot = __builtin_fmaf(x1[i], k1[i], __builtin_fmaf(x2[i], k2[i], dot));
     const float z = row16_sum(on ? dot : 0.f) * p.scale_log2;
+    // A score of -inf weighs nothing, also as the first (where z - m_new has no value); +inf and
+    // NaN make the row NaN, as do scores of -inf alone (l stays 0).
     const float m_new = fmaxf(mx, z);
-    const float alpha = __builtin_amdgcn_exp2f(mx - m_new), w = __builtin_amdgcn_exp2f(z - m_new);
+    const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mx - m_new);
+    const float w = z == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(z - m_new);
     mx = m_new;
     l = l * alpha + w;
 #pragma unroll

@@ -139,3 +139,23 @@ def test_vt_pack_of_more_slabs_than_a_grid_axis(cdx):
     nat.check(nat.lib().cdx_vt_pack(v.data_ptr(), slabs, rows, S, D, vt.data_ptr(), vt.shape[-1], nat.stream_of(v)),
               "cdx_vt_pack")
     assert torch.equal(vt, to_vt_layout(v[:, :, :S].contiguous()))
+
+
+def test_a_score_of_minus_infinity_in_a_step(cdx):
+    """An infinite value in a cached key gives scores of -inf (no weight: the row stays finite
+    while another key has one) or +inf (NaN), as softmax does."""
+    print("kv cache: infinite keys", flush=True)
+    m = _module(cdx, 1, 1, 64, seed=5)
+    g = torch.Generator().manual_seed(6)
+    new = lambda *s: torch.randn(*s, generator=g).to(bf16).cuda()  # noqa: E731
+    B, S, past = 12, 5, 9  # (at most 64 rows: the pass over the cache attends itself)
+    x, kv = new(B, S, 64), [new(B, 1, past, 64), new(B, 1, past, 64)]
+    kv[0][:, :, 0, 3] = math.inf
+    kv[0][::2, :, 2, 3] = math.inf
+    with torch.no_grad():
+        out, _ = m(x, past_key_value=kv, use_cache=True)
+    ref, _, _ = _reference(m, x, None, kv)
+    finite = torch.isfinite(ref).all(-1)
+    assert 0 < int(finite.sum()) < B * S and bool(finite[1::2, 1:].any())
+    assert torch.equal(torch.isfinite(out).all(-1).cpu(), finite)
+    assert_close_bf16(out.cpu()[finite], ref[finite], "finite rows")
