@@ -179,8 +179,11 @@ class TransformerBlock(nn.Module):
         not the plain one (a replaced or hooked submodule or method, a dense MLP) or the
         operands are not the usual ones."""
         fast = nat.host()
-        attn, mlp = self.self_attn, self.mlp
-        ln1, ln2 = self.input_layernorm, self.post_attention_layernorm
+        # (Read from _modules: nn.Module's attribute search takes half a microsecond a name, more
+        # than the comparisons that decide here.)
+        mods = self._modules
+        attn, mlp = mods["self_attn"], mods["mlp"]
+        ln1, ln2 = mods["input_layernorm"], mods["post_attention_layernorm"]
         cls, own = type(self), self.__dict__
         if (fast is None or route is None or cls.forward_fused is not _FORWARD_FUSED or cls._mlp is not _MLP
                 or "forward_fused" in own or "_mlp" in own
