@@ -15,6 +15,8 @@
 //                        read and clamped in the epilogue)
 //   cdx_linear_fwd       y = x @ W^T (the tied LM head)
 // Products of up to 64 rows (a generation step) run on the skinny kernels (cdx_skinny.h).
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "cdx_gemm_persist.h"
@@ -52,36 +54,67 @@ using Small2Cfg = GemmCfg<128, 64, 2, 2, 2, 1, 1, 128>;
 using NarrowHeadCfg = GemmCfg<128, 64, 3, 1, 4, 1, 1, kBM, 1>;
 using SmallHeadCfg = GemmCfg<128, 64, 3, 1, 2, 1, 1, 128, 1>;
 
+// Row tiles of `rows` rows that a grouped pass of T rows over E experts is likely to have: half
+// a partial tile per expert beside the whole ones, but no more than even segments give, their
+// length taken `sigmas` standard deviations long (T / E rows of each expert are a binomial's
+// mean), and one tile per expert at least.  (The host does not read the plan.  Segments of very
+// different lengths have up to E / 2 more.)
+int64_t grouped_row_tiles(int64_t T, int64_t E, int64_t rows, double sigmas) {
+  const double s = (double)T / (double)E;
+  const int64_t even = E * (int64_t)std::ceil((s + sigmas * std::sqrt(s)) / (double)rows);
+  return std::max(std::min(E, T), std::min((T + rows - 1) / rows + (E + 1) / 2, even));
+}
+
 // The tile for products of a size between one 128-row tile per CU and whole rounds of
-// 256 x 256 tiles.  0: the 256-row forms, 1: XSmallCfg, 2: SmallCfg, 3: Small2Cfg.  Grouped
-// passes count half a partial tile per expert.
+// 256 x 256 tiles.  0: the 256-row forms, 1: XSmallCfg, 2: SmallCfg, 3: Small2Cfg.
 // Plain epilogues: the smallest tile that leaves at most one tile per CU (128 x 64 tiles at
-// two per CU lose to 128 x 128 ones at one: their LDS reads per MFMA are half as many again),
-// then two 128 x 128 tiles per CU.  One 256-row tile of M reads B once, so few rows stay with
-// the 256-row forms.  us, before -> here: mu guidance 2048 x 768 8.1 -> 8.1 (128 x 64), 3000 x
-// 1280 16.8 -> 15.4 (128 x 128), 4096 x 2048 35.4 -> 32.6 (two per CU); linear 1554 x 2560 x
-// 1920 27.3 -> 22.3; 200 x 768 x 32000 stays at 19.8 (two per CU: 22.4); MoE down passes 3001 x
-// 1792 x 1280 29.2 -> 27.6 (one tile per CU 21.6 while all fit one round, 33 with four over),
-// 6000 rows 46.8 -> 30.6, 12000 rows stay at 51 (two per CU: 66).
+// two per CU lose to 128 x 128 ones at one: their LDS reads per MFMA are half as many again).
+// us, the 256-row forms -> here: mu guidance 2048 x 768 8.1 -> 8.1 (128 x 64), 3000 x 1280 16.8
+// -> 15.4 (128 x 128); linear 1554 x 2560 x 1920 27.3 -> 22.3; MoE down pass of 3001 x 1792 x 1280
+// 29.2 -> 27.6.
+// Up to two 128 x 128 tiles per CU then run as such
+//   * where the 256-row form would be 256 x 256 tiles on part of the chip, i.e. the 256 x 128
+//     ones take more than a round: 1.3 to 1.5 times as fast at any K (grouped: 6000 x 1792 x 1280
+//     46.8 -> 30.6), and
+//   * for short products, whose prologues and epilogues the second block hides: K <= 768 and
+//     weights up to 5 MB (1.06 to 1.2 times as fast with the weights in cache; from HBM 1.0 to 1.2,
+//     at K = 768 and 2048 or 4096 rows 0.88 to 0.94).  Beyond, a pair's K step is the longer one,
+//     1.02 us against 0.79: 2048 x 2048 x 4096 33.2 and 38.8, 4096 x 1536 x 1536 0.92 from HBM.
+//     mu-QKV + RoPE to K = 2048: 1.06 to 1.17 with the weights in cache, 0.89 to 1.01 from HBM; a
+//     150M forward of 3547 to 6000 tokens 1-2% faster, of 4096 0.8% slower.
+//     Grouped passes gain at any K, but for 1.2 to 1.6 tiles a CU (0.92 to 0.99).
+// One 256-row tile of M reads B once, so few rows stay with the 256-row forms (200 x 768 x 32000
+// 19.8, two per CU 22.4).
 // SwiGLU: one 128 x 128 tile per CU where that is all (400 tokens, 2048 wide: 30.9 -> 18.1),
-// else the cheaper of two tiles per CU, per tile 0.42 us a K step + 2.5, and rounds of
-// 256 x 256 tiles, 1.2 us a K step + 8 (fitted to 13 shapes within 15%): 2048 x 768 16.6 ->
-// 14.5, 8192 x 768 44.0 -> 36.9, 1000 x 2048 42.0 -> 26.4, 2048 x 2048 44.3 -> 30.9; 3001 x 1280 stays at 33.8 (36.1).
+// else the cheaper of pairs of them, 0.9 us a K step + 4 (0.5 + 4 for one left over), and rounds of
+// 256 x 256 tiles, 1.1 us a K step + 10.  (A price per tile without the whole rounds sent 3001
+// tokens of 2048 to pairs that take 13 us longer.)
+// All MoE shapes of 256 to 8192 wide, 65 to 12000 tokens and 4 to 64 experts, 242 in all, against
+// the 256-row forms: 1.12 times as fast (geometric mean), one slower by more than 3% (0.96); with
+// 90% of the tokens in one expert, whose tiles the host cannot count, 1.08 and twelve (to 0.80).
 template <ALoad AL, Epi EP, int HD>
 int mid_tile(const GemmParams& p) {
   if (AL == ALoad::kSegmented || (EP == Epi::kQKRope && HD == 128)) return 0;
-  const int64_t cus = device_cu_count(), half_e = p.offsets != nullptr ? (p.E + 1) / 2 : 0;
-  const int64_t m128 = (p.M + 127) / 128 + half_e, n128 = (p.N + 127) / 128, t128 = m128 * n128;
+  const int64_t cus = device_cu_count();
+  const bool grouped = p.offsets != nullptr;
+  const int64_t m128 = grouped ? grouped_row_tiles(p.M, p.E, 128, 3) : (p.M + 127) / 128;
+  const int64_t t128 = m128 * ((p.N + 127) / 128), n256 = (p.N + 255) / 256;
   if (EP == Epi::kSwiGLU) {
     if (t128 <= cus) return 2;
-    const int64_t t256 = ((p.M + 255) / 256 + half_e) * ((p.N + 255) / 256);
-    const double kt = p.K / 64, n = (double)t128 / cus;
-    const double two = n * (0.42 * kt + 2.5) + 5, square = (double)((t256 + cus - 1) / cus) * (1.2 * kt + 8);
-    return two < square ? 3 : 0;
+    const int64_t t256 = (grouped ? grouped_row_tiles(p.M, p.E, 256, 1) : (p.M + 255) / 256) * n256;
+    const int64_t per_cu = (t128 + cus - 1) / cus;
+    const double kt = p.K / 64;
+    const double pairs = (double)(per_cu / 2) * (0.9 * kt + 4) + (double)(per_cu % 2) * (0.5 * kt + 4);
+    return pairs < (double)((t256 + cus - 1) / cus) * (1.1 * kt + 10) ? 3 : 0;
   }
   if (EP != Epi::kQKRope && m128 * ((p.N + 63) / 64) <= cus) return 1;
   if (t128 <= cus) return 2;
-  return t128 <= 2 * cus && (p.M > kBM || p.offsets != nullptr) ? 3 : 0;
+  if (t128 > 2 * cus || (p.M <= kBM && !grouped)) return 0;
+  // 2 x the 256 x 256 tiles that `launch` counts: the 256 x 128 ones.
+  if (2 * p.mt_count * n256 > cus) return 3;
+  if (grouped) return 5 * t128 > 6 * cus && 5 * t128 < 8 * cus ? 0 : 3;
+  if (EP == Epi::kQKRope) return p.K <= 2048 ? 3 : 0;
+  return p.K <= 768 && (int64_t)p.K * p.N <= 5 << 19 ? 3 : 0;
 }
 
 template <ALoad AL, Epi EP, class Cfg = DefaultCfg, int HD = 0>
@@ -304,8 +337,7 @@ int moe_swiglu(const uint16_t* x, int64_t T, int32_t H, int32_t Ie, int32_t E, i
   const int64_t cost_expert = cdiv((cdiv(T, kBM) + E - 1) * nt2, cus) * (ks_shared + ks_expert);
   const int64_t cost_segmented = cdiv(cdiv(T, kBM) * nt2, cus) * (ks_shared + ks_expert) + ks_expert;
   // (Up to two 128 x 128 per-expert tiles per CU run as such, see mid_tile.)
-  const bool segmented = cost_segmented < cost_expert &&
-                         (cdiv(T, 128) + (E + 1) / 2) * cdiv(H, 128) > 2 * cus;
+  const bool segmented = cost_segmented < cost_expert && grouped_row_tiles(T, E, 128, 3) * cdiv(H, 128) > 2 * cus;
   // B: w_down [blocks][H][P]; the shared block (if any) serves K columns [0, P), the
   // token's expert block K columns [k_split, K).
   GemmParams p2{};
