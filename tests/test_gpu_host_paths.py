@@ -243,3 +243,30 @@ def test_linear_accumulate_checks_every_size(cdx):
                     linear_accumulate_(x, weight, res)
             finally:
                 nat.set_launch_hook(None)
+
+
+@pytest.mark.parametrize("B,S,past", [(2, 1, 4), (1, 7, 7), (1, 8, 0)])
+def test_block_step_of_a_wide_projection(cdx, B, S, past):
+    """9216 columns of q, k and v (3072 wide, as many KV heads as query heads): the folded norm on
+    the blocks of 32 output columns, which the narrower projections of test_block_step do not take."""
+    from complexity_deep.normalization import rms_norm
+    print(f"block step, wide projection B={B} S={S} past={past}", flush=True)
+    H, heads, D = 3072, 24, 128
+    torch.manual_seed(S)
+    blk = cdx.TransformerBlock(H, 1024, heads, heads, num_experts=2, vocab_size=500,
+                               use_mu_guidance=False).to(bf16).cuda().eval()
+    with torch.no_grad():
+        blk.input_layernorm.weight.normal_(1, 0.2)
+    ids = torch.randint(0, 500, (B, S), device="cuda")
+    kv = (_new(B, heads, past, D), _new(B, heads, past, D, seed=1)) if past else None
+    mu, h = _new(B, S, H, seed=5), _new(B, S, H)
+    nxt = cdx.RMSNorm(H).to(bf16).cuda()
+    with torch.no_grad():
+        plan = blk.mlp.plan(ids)
+        a, b = h.clone(), h.clone()
+        (k, v), none = blk.step(a, mu, kv, plan)
+        _, _, kv_b, _ = blk.forward_fused(b, rms_norm(b, blk.input_layernorm.weight, 1e-6), nxt, past_key_value=kv,
+                                          use_cache=True, token_ids=ids, mu_prev=mu, route=plan)
+    assert none is None
+    for x, y, what in ((a, b, "h"), (k, kv_b[0], "k"), (v, kv_b[1], "v")):
+        _near(x, y, what)

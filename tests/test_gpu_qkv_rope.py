@@ -240,8 +240,8 @@ def test_qkv_rope_many_tiles(cdx, oracle, B, S, H, nq, nkv, mu_mode, pos0, qk_no
                                           (16, 1024, 2048, 16, 8)])  # D = 128: 256 x 256 vs persistent
 def test_qkv_rope_sequences_independent_of_batch(cdx, B, S, H, nq, nkv):
     """A sequence's q, k and V^T do not depend on the rest of the batch: the first two
-    sequences alone (few tiles: the 128-row tiles at head dim 64, one 256 x 256 tile per
-    block at 128) and inside a batch of B (256-row tiles, the persistent form at head dim
+    sequences alone (few tiles: the 128-row tiles at head dim 64, 128-column tiles at 128)
+    and inside a batch of B (256-row tiles, the persistent form at head dim
     128) give the same bits.  Every tile form accumulates an element over K in the same
     order and runs the same QK-norm + RoPE arithmetic."""
     from complexity_deep.attention import mu_qkv_rope
