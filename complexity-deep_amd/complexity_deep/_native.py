@@ -110,7 +110,9 @@ def lib():
 
 # Optional per-call timing hook: when set, every C-ABI launch site records a pair of
 # timing events on the stream the kernels go to and hands them to the hook as
-# hook(name, start_event, end_event, shape_dict).  None (the default) costs one test.
+# hook(name, start_event, end_event, shape_dict).  None (the default) costs one test.  While a
+# hook is set the operators take their Python launch sites: the same kernels, except that a
+# prompt's V^T has its own launch and that a step of up to 8 rows runs with separate norms.
 _launch_hook: Optional[Callable] = None
 
 

@@ -198,7 +198,7 @@ class ComplexityModel(nn.Module):
 
     def route_plans(self, input_ids: torch.Tensor) -> List[Optional[RoutePlan]]:
         """One routing plan per routed layer, each through the layer's own map: every
-        plan of the forward in one cdx_route_plans call (two launches), with no host
+        plan of the forward in one cdx_route_plans call (one launch, two past 4096 ids), with no host
         synchronisation.  Layers whose MLPs differ in expert count or vocabulary get
         a call per kind."""
         out: List[Optional[RoutePlan]] = [None] * len(self.layers)

@@ -1,8 +1,8 @@
 """Rotary position embedding; interface of core/rotary.py:16-86.
 
-Used around the QKV projection but not one of the three kernel pieces: it runs as
-PyTorch ops on the GPU.  ``inv_freq`` is a persistent buffer (it is in the
-reference's state_dict); the cos/sin tables are non-persistent and grow on demand.
+The kernels rotate by ``cos_sin_table`` (fp32); ``forward``'s tables serve the PyTorch path
+(head dims or masks that the kernels do not take).  ``inv_freq`` is a persistent buffer (it
+is in the reference's state_dict); the tables are non-persistent and grow on demand.
 
 Angles are always formed in fp32 from the exact fp32 inverse frequencies, computed
 from ``dim`` and ``theta`` the way the reference's constructor computes them

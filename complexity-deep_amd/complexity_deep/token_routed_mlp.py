@@ -95,7 +95,7 @@ def route_plan(ids: torch.Tensor, token_map: Optional[torch.Tensor], num_experts
 
 def route_plans(ids: torch.Tensor, token_maps: Sequence[torch.Tensor], num_experts: int) -> List[RoutePlan]:
     """One bit-exact routing plan per map over the same ids (cdx_route_plans): plan y
-    routes through token_maps[y], all of them in the same two launches.  Every map is
+    routes through token_maps[y], all of them in the same launch (two past 4096 ids).  Every map is
     int64 [V] with one V for all; ids as in route_plan.  Plan y's tensors are rows of
     [L, ...] buffers and equal route_plan(ids, token_maps[y], num_experts)."""
     L = len(token_maps)

@@ -532,6 +532,10 @@ int skinny_gemm(const SkinnyParams& p, SkinnyEpi epi, hipStream_t s, const char*
     return fail(CDX_EUNSUPPORTED, "%s: a folded norm needs M <= 8", name);
   // The columns per block grow with N: one MFMA's worth while that fills the chip at most
   // once, more for wider outputs (fewer blocks and A reads for the same loads in flight).
+  // us on 256 CUs, weights from HBM.  8 rows, K = 2048, blocks of 8 / 16 / 32 columns: N = 2048 4.7 /
+  // 5.5 / 7.2, 4096 6.5 / 6.0 / 7.5, 8192 10.3 / 9.1 / 10.0, 32000 35.0 / 30.0 / 30.7 (K = 768: 16.2 /
+  // 13.3 / 12.0).  16 rows, blocks of 16 / 64: N = 4096 6.5 / 11.9, 8192 10.4 / 12.7, 12288 14.9 / 14.0,
+  // 32000 35.9 / 33.2.
   if (p.M <= 8) {
     if (p.N <= 8 * cus) return launch_skinny<1, 1, 8, 8, true>(p, epi, s, name);
     if (p.N <= 32 * cus) return launch_skinny<1, 2, 8, 4, true>(p, epi, s, name);

@@ -3,7 +3,8 @@
 // A forward of few tokens is paced by its host side: checks, output tensors and ctypes
 // conversions in Python took 6 to 20 us per operator against 2 to 10 us of kernel time.
 // Measured (us per call, issued back to back): 1B attention step of 4 rows 46 -> 22, MoE step
-// 32 -> 21, 150M model step 1360 -> 762, 150M block of 2048 tokens 148 -> 90.
+// 32 -> 21, 150M block of 2048 tokens 148 -> 90, 150M model step 1360 -> 762 (with block_step
+// 510).
 // Each function here is the usual case of one Python operator of the same name: it checks
 // its operands, allocates the outputs through torch's allocator, and calls the C-ABI on the
 // current stream.  For anything else (a tensor to be made contiguous, cast or broadcast, a
