@@ -82,16 +82,17 @@ int64_t grouped_row_tiles(int64_t T, int64_t E, int64_t rows, double sigmas) {
 //     1.02 us against 0.79: 2048 x 2048 x 4096 33.2 and 38.8, 4096 x 1536 x 1536 0.92 from HBM.
 //     mu-QKV + RoPE to K = 2048: 1.06 to 1.17 with the weights in cache, 0.89 to 1.01 from HBM; a
 //     150M forward of 3547 to 6000 tokens 1-2% faster, of 4096 0.8% slower.
-//     Grouped passes gain at any K, but for 1.2 to 1.6 tiles a CU (0.92 to 0.99).
+//     Grouped passes gain at any K, but past K = 512 not with 1.2 to 1.6 tiles a CU (0.92 to 0.99;
+//     12000 x 256 x 512 9.8 -> 8.1).
 // One 256-row tile of M reads B once, so few rows stay with the 256-row forms (200 x 768 x 32000
 // 19.8, two per CU 22.4).
 // SwiGLU: one 128 x 128 tile per CU where that is all (400 tokens, 2048 wide: 30.9 -> 18.1),
-// else the cheaper of pairs of them, 0.9 us a K step + 4 (0.5 + 4 for one left over), and rounds of
+// else the cheaper of pairs of them, 0.9 us a K step + 4 (0.5 + 2 for one left over), and rounds of
 // 256 x 256 tiles, 1.1 us a K step + 10.  (A price per tile without the whole rounds sent 3001
 // tokens of 2048 to pairs that take 13 us longer.)
 // All MoE shapes of 256 to 8192 wide, 65 to 12000 tokens and 4 to 64 experts, 242 in all, against
-// the 256-row forms: 1.12 times as fast (geometric mean), one slower by more than 3% (0.96); with
-// 90% of the tokens in one expert, whose tiles the host cannot count, 1.08 and twelve (to 0.80).
+// the 256-row forms: 1.12 times as fast (geometric mean), one slower by more than 3% (0.95); with
+// 90% of the tokens in one expert, whose tiles the host cannot count, 1.08 and eleven (to 0.80).
 template <ALoad AL, Epi EP, int HD>
 int mid_tile(const GemmParams& p) {
   if (AL == ALoad::kSegmented || (EP == Epi::kQKRope && HD == 128)) return 0;
@@ -104,7 +105,7 @@ int mid_tile(const GemmParams& p) {
     const int64_t t256 = (grouped ? grouped_row_tiles(p.M, p.E, 256, 1) : (p.M + 255) / 256) * n256;
     const int64_t per_cu = (t128 + cus - 1) / cus;
     const double kt = p.K / 64;
-    const double pairs = (double)(per_cu / 2) * (0.9 * kt + 4) + (double)(per_cu % 2) * (0.5 * kt + 4);
+    const double pairs = (double)(per_cu / 2) * (0.9 * kt + 4) + (double)(per_cu % 2) * (0.5 * kt + 2);
     return pairs < (double)((t256 + cus - 1) / cus) * (1.1 * kt + 10) ? 3 : 0;
   }
   if (EP != Epi::kQKRope && m128 * ((p.N + 63) / 64) <= cus) return 1;
@@ -112,7 +113,7 @@ int mid_tile(const GemmParams& p) {
   if (t128 > 2 * cus || (p.M <= kBM && !grouped)) return 0;
   // 2 x the 256 x 256 tiles that `launch` counts: the 256 x 128 ones.
   if (2 * p.mt_count * n256 > cus) return 3;
-  if (grouped) return 5 * t128 > 6 * cus && 5 * t128 < 8 * cus ? 0 : 3;
+  if (grouped) return p.K > 512 && 5 * t128 > 6 * cus && 5 * t128 < 8 * cus ? 0 : 3;
   if (EP == Epi::kQKRope) return p.K <= 2048 ? 3 : 0;
   return p.K <= 768 && (int64_t)p.K * p.N <= 5 << 19 ? 3 : 0;
 }
